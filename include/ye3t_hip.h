@@ -7,7 +7,8 @@
  *     (host pointers only where a comment says "host").
  *   - `dtype` is YE3T_F32 or YE3T_F64; float arrays of one call share it.
  *   - Work is enqueued on `stream` (NULL = default stream); calls never
- *     synchronise the device except plan creation, which copies tables.
+ *     synchronise the device except plan creation, which copies tables, and
+ *     ye3t_hip_check_indices, which waits for its answer.
  *   - Return 0 on success, a negative ye3t_status on failure; the message of
  *     the last failure on the calling thread is ye3t_hip_last_error().
  *     Nothing throws across this boundary.
@@ -125,6 +126,22 @@ int ye3t_hip_density_accumulate_csr(int dtype, const void* edge_values, const in
 int ye3t_hip_density_accumulate_adjoint(int dtype, const void* atomic_adjoint, const int64_t* centers,
                                         int64_t edge_count, int64_t channel_count, int64_t atom_count,
                                         void* edge_adjoint, ye3t_stream_t stream);
+
+/* Checks index inputs on the device in one pass and waits for the answer.
+ * row_offsets (NULL: not checked) has atom_count + 1 entries, indices (NULL:
+ * not checked) index_count entries to lie in [0, index_limit), species (NULL:
+ * not checked) atom_count entries to lie in [0, species_count).  result (host,
+ * YE3T_CHECK_RESULTS words) receives: [0] row_offsets[0]; [1]
+ * row_offsets[atom_count]; then 1 for each fault, else 0: [2] row_offsets fall
+ * somewhere, [3] an index is out of range, [4] a species is out of range, [5]
+ * without row_offsets, the indices fall somewhere.  Synchronises `stream`;
+ * YE3T_EUNSUPPORTED, with nothing launched, while the stream is captured.
+ * Replaces the host guards in front of the reference's gathers
+ * (execution_plan_cuda.cu:37-197). */
+#define YE3T_CHECK_RESULTS 6
+int ye3t_hip_check_indices(const int64_t* row_offsets, int64_t atom_count, const int64_t* indices,
+                           int64_t index_count, int64_t index_limit, const int32_t* species, int64_t species_count,
+                           int64_t* result, ye3t_stream_t stream);
 
 /* Fused stage 1: A[i, c, r, lm] = sum_{e in row i} w_c(e) R_r(|v_e|) Y_lm(v_e/|v_e|).
  * One pass over edges: radial basis and real SH in registers, per-atom CSR

@@ -1,0 +1,60 @@
+"""The device check of index inputs against the same conditions in Torch."""
+
+import pytest
+
+from tests._util import flush
+
+pytestmark = pytest.mark.gpu
+
+
+def _expect(offsets, indices, limit, species, kinds):
+    return [int(offsets[0]), int(offsets[-1]), int(bool((offsets[1:] < offsets[:-1]).any())),
+            int(bool(((indices < 0) | (indices >= limit)).any())),
+            int(bool(((species < 0) | (species >= kinds)).any())), 0]
+
+
+@pytest.mark.parametrize("atoms,edges", [(1, 1), (5, 0), (3, 255), (300, 257), (2049, 70001), (70001, 513)])
+def test_check_indices_finds_each_fault_at_every_end(gpu, atoms, edges):
+    """No fault in clean input; each kind of fault at the first, middle and last place is found, and only that kind."""
+    flush(f"index checks, {atoms} atoms, {edges} edges")
+    import torch
+
+    from ye3t_amd.runtime import native, validate_density_csr
+
+    g = torch.Generator().manual_seed(atoms)
+    cuts = torch.sort(torch.randint(0, edges + 1, (atoms - 1,), generator=g)).values
+    offsets = torch.cat([torch.zeros(1, dtype=torch.int64), cuts, torch.tensor([edges])]).to(gpu)
+    nbr = torch.randint(0, atoms, (edges,), generator=g).to(gpu)
+    species = torch.randint(0, 4, (atoms,), generator=g).to(gpu, torch.int32)
+
+    def look(o, n, s):
+        got = native.check_indices(o, atoms, n, atoms, s, 4)
+        assert got == _expect(o.cpu(), n.cpu(), atoms, s.cpu(), 4)
+        return got
+
+    assert look(offsets, nbr, species)[2:] == [0, 0, 0, 0]
+    assert validate_density_csr(offsets, nbr, atoms, edges, species=species, species_count=4)
+    for at in {0, edges // 2, edges - 1} if edges else ():
+        for value in (-1, atoms, 2 ** 40):
+            bad = nbr.clone()
+            bad[at] = value
+            assert look(offsets, bad, species)[3] == 1
+            with pytest.raises(ValueError, match="neighbor index"):
+                validate_density_csr(offsets, bad, atoms, edges)
+    for at in {0, atoms // 2, atoms - 1}:
+        for value in (-1, 4):
+            bad = species.clone()
+            bad[at] = value
+            assert look(offsets, nbr, bad)[4] == 1
+            with pytest.raises(ValueError, match="species index"):
+                validate_density_csr(offsets, nbr, atoms, edges, species=bad, species_count=4)
+        bad = offsets.clone()
+        bad[at] = edges + 1
+        assert look(bad, nbr, species)[2] == 1
+        with pytest.raises(ValueError, match="row_offsets"):
+            validate_density_csr(bad, nbr, atoms, edges)
+    # what the device cannot look at: other layouts keep the Torch checks
+    if edges > 1:
+        strided = torch.stack([nbr, nbr], dim=1)[:, 0]
+        assert native.check_indices(offsets, atoms, strided, atoms) is None
+        assert validate_density_csr(offsets, strided, atoms, edges)

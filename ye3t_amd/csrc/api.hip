@@ -259,6 +259,55 @@ __global__ __launch_bounds__(256) void density_adjoint_kernel(const V* __restric
   }
 }
 
+// Range checks of a density's index inputs in one pass over them: nothing is
+// reduced, a lane that sees a violation stores its word of `status` (host
+// memory the device can write, zeroed by the host), and the first and last
+// offsets are copied there.  A structure of 50 000 atoms and 1.2 M edges is
+// 10 MB, about 4 us of reads; taken as torch reductions with a read-back each
+// (minimum and maximum of the neighbours, first and last offset, monotony) the
+// same checks are six kernels and five synchronisations: a 16-channel density
+// and product of 50 000 atoms took 260 us with those, 169 us with this, and
+// one of 128 atoms 110 and 40 us.
+template <typename T>
+__device__ inline void check_range(const T* __restrict__ v, int64_t n, int64_t limit, bool ordered,
+                                   int64_t* __restrict__ bad, int64_t* __restrict__ descends) {
+  const int64_t stride = int64_t(gridDim.x) * blockDim.x;
+  for (int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < n; k += stride) {
+    const int64_t x = int64_t(v[k]);
+    if (x < 0 || x >= limit) *bad = 1;
+    if (ordered && k > 0 && int64_t(v[k - 1]) > x) *descends = 1;
+  }
+}
+
+__global__ __launch_bounds__(256) void check_indices_kernel(const int64_t* __restrict__ offsets, int64_t N,
+                                                            const int64_t* __restrict__ indices, int64_t count,
+                                                            int64_t limit, const int32_t* __restrict__ species,
+                                                            int64_t species_count, int64_t* __restrict__ status) {
+  if (offsets != nullptr) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      status[0] = offsets[0];
+      status[1] = offsets[N];
+    }
+    const int64_t stride = int64_t(gridDim.x) * blockDim.x;
+    for (int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < N; k += stride)
+      if (offsets[k] > offsets[k + 1]) status[2] = 1;
+  }
+  if (indices != nullptr) check_range(indices, count, limit, offsets == nullptr, status + 3, status + 5);
+  if (species != nullptr) check_range(species, N, species_count, false, status + 4, status + 6);
+}
+
+// The status words of the calling thread: pinned host memory, made at the
+// thread's first check and freed when the thread ends.  A check waits for its
+// kernel before it returns, so one set per thread is enough for any number of
+// streams.
+struct CheckStatus {
+  int64_t* words = nullptr;
+  ~CheckStatus() {
+    if (words != nullptr) (void)hipHostFree(words);
+  }
+};
+constexpr int kCheckWords = 8;
+
 inline unsigned grid_for(int64_t work, int threads) {
   int64_t g = (work + threads - 1) / threads;
   if (g < 1) g = 1;
@@ -402,6 +451,38 @@ int ye3t_hip_density_accumulate_csr(int dtype, const void* ev, const int64_t* of
     return set_error(YE3T_EDTYPE, "unsupported dtype %d", dtype);
   }
   return check_launch("density_csr_kernel");
+}
+
+int ye3t_hip_check_indices(const int64_t* row_offsets, int64_t atom_count, const int64_t* indices, int64_t index_count,
+                           int64_t index_limit, const int32_t* species, int64_t species_count, int64_t* result,
+                           ye3t_stream_t stream) {
+  clear_error();
+  YE3T_REQUIRE(atom_count >= 0 && index_count >= 0, "negative size");
+  YE3T_REQUIRE(result != nullptr, "NULL result");
+  const hipStream_t s = as_stream(stream);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  YE3T_CHECK_HIP(hipStreamIsCapturing(s, &capture));
+  if (capture != hipStreamCaptureStatusNone)
+    return set_error(YE3T_EUNSUPPORTED, "indices cannot be checked while the stream is captured");
+  static thread_local CheckStatus status;
+  if (status.words == nullptr) {
+    void* words = nullptr;
+    YE3T_CHECK_HIP(hipHostMalloc(&words, kCheckWords * sizeof(int64_t), hipHostMallocPortable | hipHostMallocMapped));
+    status.words = static_cast<int64_t*>(words);
+  }
+  for (int k = 0; k < kCheckWords; ++k) status.words[k] = 0;
+  // eight indices per lane and pass: enough wavefronts to cover the latency of a
+  // short read, and few enough workgroups for the smallest calls to start at once
+  const int64_t most = index_count > atom_count ? index_count : atom_count;
+  const unsigned grid = grid_for((most + 7) / 8, 256);
+  hipLaunchKernelGGL(check_indices_kernel, dim3(grid), dim3(256), 0, s, row_offsets, atom_count,
+                     index_count > 0 ? indices : nullptr, index_count, index_limit,
+                     atom_count > 0 ? species : nullptr, species_count, status.words);
+  const int rc = check_launch("check_indices_kernel");
+  if (rc != YE3T_OK) return rc;
+  YE3T_CHECK_HIP(hipStreamSynchronize(s));
+  for (int k = 0; k < YE3T_CHECK_RESULTS; ++k) result[k] = status.words[k];
+  return YE3T_OK;
 }
 
 int ye3t_hip_density_accumulate_adjoint(int dtype, const void* adj, const int64_t* centers, int64_t E, int64_t C,

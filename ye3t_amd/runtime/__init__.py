@@ -246,6 +246,21 @@ def scheduled_radial_angular_channels_with_derivative(radial_values, radial_deri
                                                     channel_scales)
 
 
+def _csr_passes(row_offsets, neighbors, atom_count, edge_count, species, species_count):
+    """Whether the device finds nothing to object to in these index inputs."""
+    import torch
+
+    shaped = row_offsets.dtype == torch.int64 and row_offsets.shape == (atom_count + 1,) and (
+        neighbors is None or (neighbors.dtype == torch.int64 and neighbors.shape == (edge_count,))) and (
+        species is None or (species.dtype == torch.int32 and species.shape == (atom_count,)
+                            and species_count is not None))
+    if not shaped:
+        return False
+    found = native.check_indices(row_offsets, atom_count, neighbors, atom_count, species,
+                                 0 if species is None else int(species_count))
+    return found is not None and found[0] == 0 and found[1] == edge_count and not any(found[2:5])
+
+
 def validate_density_csr(row_offsets, neighbors, atom_count, edge_count, *, species=None, species_count=None):
     """Host-side range checks of the fused density's index inputs (any device).
 
@@ -254,12 +269,16 @@ def validate_density_csr(row_offsets, neighbors, atom_count, edge_count, *, spec
     ``species`` int32 ``[N]`` in ``[0, species_count)``.  The kernels gather
     through these indices without bounds checks, as the reference's do after
     its own ``TORCH_CHECK`` guards (``execution_plan_cuda.cu:37-197``), so bad
-    indices raise here before any launch.  Each check reduces on the tensor's
-    device and reads one scalar back.
+    indices raise here before any launch.  Tensors on the GPU are checked by
+    one kernel and one wait (``native.check_indices``); where that finds a
+    fault, or cannot look, each check reduces on the tensor's device and reads
+    one scalar back, and names it.
     """
     import torch
 
     atom_count, edge_count = int(atom_count), int(edge_count)
+    if row_offsets.is_cuda and _csr_passes(row_offsets, neighbors, atom_count, edge_count, species, species_count):
+        return True
     if row_offsets.dtype != torch.int64 or tuple(row_offsets.shape) != (atom_count + 1,):
         raise ValueError(f"row_offsets must be int64 [{atom_count + 1}]")
     first, last = int(row_offsets[0]), int(row_offsets[-1])

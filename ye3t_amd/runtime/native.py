@@ -16,6 +16,7 @@ ABI_VERSION = 61
 _LIB = None
 
 F32, F64 = 0, 1
+EUNSUPPORTED = -5
 
 _vp = ctypes.c_void_p
 _i64 = ctypes.c_int64
@@ -105,6 +106,7 @@ def lib():
     L.ye3t_hip_scheduled_radial_angular_channels.argtypes = [ctypes.c_int, _i64, _i64, _i64, _i64] + [_vp] * 13
     L.ye3t_hip_density_accumulate_csr.argtypes = [ctypes.c_int, _vp, _vp, _i64, _i64, _vp, _vp]
     L.ye3t_hip_density_accumulate_adjoint.argtypes = [ctypes.c_int, _vp, _vp, _i64, _i64, _i64, _vp, _vp]
+    L.ye3t_hip_check_indices.argtypes = [_vp, _i64, _vp, _i64, _i64, _vp, _i64, ctypes.POINTER(_i64), _vp]
     L.ye3t_hip_ace_density_forward.argtypes = [ctypes.POINTER(DensityArgs), _vp, _vp]
     L.ye3t_hip_ace_density_edge_gradient.argtypes = [ctypes.POINTER(DensityArgs), ctypes.c_int, _vp, _vp, _vp]
     L.ye3t_hip_symmetric_power_monomial.argtypes = [ctypes.c_int, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _i64, _i64,
@@ -223,7 +225,7 @@ EXPORTED_SYMBOLS = (
     "ye3t_hip_ace_density_edge_gradient", "ye3t_hip_symmetric_power_shared_sparse_monomial",
     "ye3t_hip_symmetric_power_shared_sparse_monomial_adjoint",
     "ye3t_hip_symmetric_power_shared_sparse_monomial_double_backward", "ye3t_hip_code_object_kernel_info",
-    "ye3t_hip_part_private_limit",
+    "ye3t_hip_part_private_limit", "ye3t_hip_check_indices",
 )
 
 
@@ -372,6 +374,29 @@ def real_sph_table(vectors, l_max, epsilon=1e-12, with_gradient=True):
                                          float(epsilon), _dev(values, "values"), _opt(grads, "gradients"),
                                          _stream()), "ye3t_hip_real_sph_table")
     return values, grads
+
+
+def check_indices(row_offsets, atom_count, indices, limit, species=None, species_count=0):
+    """One device pass over index inputs (``ye3t_hip_check_indices``): the list
+    ``[first offset, last offset, offsets fall, index out of range, species out
+    of range, indices fall]``, or ``None`` where the device cannot answer (a
+    tensor that is not contiguous or not on the current device, a stream under
+    capture).  Waits for the current stream."""
+    import torch
+
+    device = torch.cuda.current_device()
+    for t in (row_offsets, indices, species):
+        if t is not None and not (t.is_cuda and t.device.index == device and t.is_contiguous()):
+            return None
+    result = (_i64 * 6)()
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    rc = lib().ye3t_hip_check_indices(ptr(row_offsets), atom_count, ptr(indices),
+                                      0 if indices is None else indices.shape[0], limit, ptr(species),
+                                      species_count, result, _stream())
+    if rc == EUNSUPPORTED:
+        return None
+    _check(rc, "ye3t_hip_check_indices")
+    return list(result)
 
 
 def density_accumulate_csr(edge_values, row_offsets, atom_count):
