@@ -1,0 +1,526 @@
+// Edge-vector gradient of the stage-1 density (forces) on the fp64 matrix
+// cores, for species (and single-channel) densities.  With the adjoint block
+// g[n][k] of edge e's centre and channel (density_grad.hip states the whole
+// formula), the per-edge sums
+//
+//   t_k = sum_n R_n g[n][k],   u_k = sum_n R'_n g[n][k],   a = sum_k u_k Y_k
+//
+// are products of an [edges x n] by an [n x k] matrix that all edges of one
+// (atom, channel) group share.  The lane-per-edge kernel gathers the block once
+// per edge: 637 loads an edge at n_max 12, l_max 6, from as many cache lines as
+// a wave has groups.  Here one wave walks its atoms in chunks of whole atoms
+// with at most 64 edges together:
+//   basis    lane = edge: radial values and derivatives and harmonics, to LDS
+//            at the edge's column, columns grouped by (atom, channel);
+//   product  per group; the block comes straight from global memory in the
+//            B-operand layout, once, as full lines, requested four groups
+//            ahead; each four edges take one v_mfma_f64_4x4x4 per four radial
+//            rows and 16 components, so a group is padded to four edges and not
+//            to the sixteen of the larger shape (its average is six at eight
+//            species and 48 neighbours); t replaces Y in LDS;
+//   chain    lane = edge: the gradient of the harmonics contracted with t.
+// Measured (kernel trace): 8 species, n_max 12, l_max 6, 30 000 atoms x 48:
+// 731 us for the lane-per-edge kernel, 480 us here; 4 species, n_max 10,
+// l_max 4, 20 000 x 32: 158 and 106 us.  It is bound by one wave per SIMD
+// (two at l_max 4) working through dependent fp64 instructions: the tile, 40 KB
+// at l_max 6, limits how many are resident.  Without the block loads it takes
+// 469 us, without the products 161.  Four waves sharing a tile, each with a
+// part of the basis, the groups and the harmonics' orders, took 520-570 us
+// (barriers, and the prologue four times); with 168 or 128 registers, for three
+// or four of them per SIMD, they spilled and took 540-670 us.
+// Lane layout of the 4x4x4 product (l = lane): A[i][k] in lanes i + 4 b + 16 k
+// for every b, B[k][j] in lane j + 16 k, D[i][j] in lane j + 16 i, j < 16.
+#include <cmath>
+
+#include "common.h"
+#include "density_grad.h"
+
+namespace ye3t {
+namespace {
+
+constexpr int kGmPitch = 68;  // pitch (doubles) of the radial rows: operand reads of 4 rows x 4 columns meet no bank twice
+
+__device__ inline uint64_t gm_ballot(bool v) { return __builtin_amdgcn_ballot_w64(v); }
+
+// LDS written by some lanes of the wave is read by others
+__device__ inline void gm_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int CTRL>
+__device__ inline double gm_dpp(double x) {
+  const long long v = __builtin_bit_cast(long long, x);
+  const int lo = __builtin_amdgcn_update_dpp(0, int(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, int(v >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (long long)((uint64_t(uint32_t(hi)) << 32) | uint32_t(lo)));
+}
+
+// sum over each 16 lanes, in every one of them
+__device__ inline double gm_sum16(double x) {
+  x += gm_dpp<0xB1>(x);   // quad_perm [1, 0, 3, 2]
+  x += gm_dpp<0x4E>(x);   // quad_perm [2, 3, 0, 1]
+  x += gm_dpp<0x141>(x);  // row_half_mirror
+  x += gm_dpp<0x140>(x);  // row_mirror
+  return x;
+}
+
+template <typename G>
+__device__ inline G gm_load(__amdgpu_buffer_rsrc_t rb, unsigned voff, unsigned soff) {
+  if constexpr (sizeof(G) == 8) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rb, voff, soff, 0));
+  } else {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, voff, soff, 0));
+  }
+}
+
+// Clamps, applied where a loaded index is used and not where it is loaded (a
+// use waits for the load): out-of-range input is never dereferenced.
+__device__ inline int64_t gm_clamp(int64_t i, int64_t n) { return i < 0 ? 0 : (i >= n ? n - 1 : i); }
+
+// Up to 64 whole atoms with at most 64 edges together from edge e of atom a on,
+// or 64 edges of an atom that has more of them left.  `end` of lane j is the
+// end of atom a + j relative to e.
+struct GmChunk {
+  int64_t a, e;
+  int na, cnt;
+  int end;
+};
+
+// offsets of the atoms after a, one per lane
+template <typename In, typename G>
+__device__ inline int64_t gm_window(const GradParams<In, G>& p, int64_t a, int64_t a_end, int lane) {
+  return p.row_offsets[a + 1 + lane < a_end ? a + 1 + lane : a_end];
+}
+
+__device__ inline GmChunk gm_form(int64_t a, int64_t e, int64_t a_end, int64_t window, int64_t edges, int lane) {
+  GmChunk c;
+  c.a = a;
+  c.e = e;
+  const int64_t rel = gm_clamp(window, edges + 1) - e;  // offsets clamped into the edge array
+  c.end = rel < 0 ? 0 : (rel > 65 ? 65 : int(rel));
+  const uint64_t fits = gm_ballot(a + 1 + lane <= a_end && c.end <= 64);
+  // the fitting atoms are a prefix (the offsets rise)
+  c.na = ~fits == 0 ? 64 : __builtin_ctzll(~fits);
+  if (c.na > 0) {
+    c.cnt = __builtin_amdgcn_readlane(c.end, c.na - 1);
+  } else {
+    c.cnt = a < a_end ? 64 : 0;
+  }
+  return c;
+}
+
+template <typename In>
+struct GmEdge {
+  In x, y, z;
+  int64_t j;
+};
+
+template <typename In, typename G>
+__device__ inline GmEdge<In> gm_edge(const GradParams<In, G>& p, const GmChunk& c, int lane) {
+  // lanes past the chunk read edge 0 (no branch: their loads need no wait before the join)
+  const int64_t e = lane < c.cnt ? c.e + lane : 0;
+  GmEdge<In> r;
+  r.x = p.vec[3 * e];
+  r.y = p.vec[3 * e + 1];
+  r.z = p.vec[3 * e + 2];
+  r.j = p.neighbors ? p.neighbors[e] : 0;
+  return r;
+}
+
+
+// Y_k(u) into a row of the tile.
+template <int LMAX>
+__device__ inline void gm_values(double x, double y, double z, const NormTable& nt, double* __restrict__ row) {
+  const double sqrt2 = 1.4142135623730950488016887242096981;
+  double cr = 1.0, ci = 0.0, qmm = 1.0;
+#pragma unroll
+  for (int m = 0; m <= LMAX; ++m) {
+    if (m > 0) {
+      qmm *= double(2 * m - 1);
+      const double nr = cr * x - ci * y;
+      const double ni = cr * y + ci * x;
+      cr = nr;
+      ci = ni;
+    }
+    double q2 = 0.0, q1 = 0.0;
+#pragma unroll
+    for (int l = m; l <= LMAX; ++l) {
+      double q;
+      if (l == m) {
+        q = qmm;
+      } else if (l == m + 1) {
+        q = double(2 * m + 1) * z * qmm;
+      } else {
+        q = (double(2 * l - 1) * z * q1 - double(l + m - 1) * q2) * nt.inv[l - m];
+      }
+      q2 = q1;
+      q1 = q;
+      const double n = nt.v[l * (kMaxL + 1) + m];
+      const int base = l * l + l;
+      if (m == 0) {
+        row[base] = n * q;
+      } else {
+        const double s = sqrt2 * n * q;
+        row[base + m] = s * cr;
+        row[base - m] = -s * ci;
+      }
+    }
+  }
+}
+
+// sum_k t_k grad_u Y_k(u) (sph_gradient_dot's sum, t read from a row of the tile).
+template <int LMAX>
+__device__ inline void gm_gradient(double x, double y, double z, const NormTable& nt, const double* __restrict__ t,
+                                   double& gx, double& gy, double& gz) {
+  const double sqrt2 = 1.4142135623730950488016887242096981;
+  gx = gy = gz = 0.0;
+  double cr = 1.0, ci = 0.0, pr = 1.0, pi = 0.0;  // (x + i y)^m and ^(m-1)
+  double qmm = 1.0;
+#pragma unroll
+  for (int m = 0; m <= LMAX; ++m) {
+    if (m > 0) {
+      qmm *= double(2 * m - 1);
+      pr = cr;
+      pi = ci;
+      const double nr = cr * x - ci * y;
+      const double ni = cr * y + ci * x;
+      cr = nr;
+      ci = ni;
+    }
+    // q: Q_l^m, d: Q_l^{m+1} = dQ_l^m / dz, both by their recurrences in l
+    double q2 = 0.0, q1 = 0.0, d2 = 0.0, d1 = 0.0;
+    const double dmm = qmm * double(2 * m + 1);
+#pragma unroll
+    for (int l = m; l <= LMAX; ++l) {
+      double q, d = 0.0;
+      if (l == m) {
+        q = qmm;
+      } else if (l == m + 1) {
+        q = double(2 * m + 1) * z * qmm;
+        d = dmm;
+      } else {
+        q = (double(2 * l - 1) * z * q1 - double(l + m - 1) * q2) * nt.inv[l - m];
+        if (l == m + 2) {
+          d = double(2 * m + 3) * z * dmm;
+        } else {
+          d = (double(2 * l - 1) * z * d1 - double(l + m) * d2) * nt.inv[l - m - 1];
+        }
+      }
+      q2 = q1;
+      q1 = q;
+      d2 = d1;
+      d1 = d;
+      const double n = nt.v[l * (kMaxL + 1) + m];
+      const int base = l * l + l;
+      if (m == 0) {
+        gz += t[base] * (n * d);
+      } else {
+        const double s = sqrt2 * n;
+        const double tp = t[base + m], tm = t[base - m];
+        // grad Y_{l,+m} = s (m q pr, -m q pi, d cr); grad Y_{l,-m} = -s (m q pi, m q pr, d ci)
+        const double sq = s * double(m) * q;
+        gx += sq * (tp * pr - tm * pi);
+        gy -= sq * (tp * pi + tm * pr);
+        gz += s * d * (tp * cr - tm * ci);
+      }
+    }
+  }
+}
+
+// Radial constants of a launch, from the host.
+struct GmRadial {
+  double rc, lambda, den;  // cutoff, lambda, expm1(lambda)
+};
+
+// The radial values and derivatives of cheb_exp_cos_row for a fixed count,
+// with one sincospi and one expm1, in fewer instructions.
+template <int NRC>
+__device__ inline void gm_radial(double r, const GmRadial& c, double (&R)[NRC], double (&dR)[NRC]) {
+  const double pi = 3.141592653589793238462643383279502884;
+  const double s = r / c.rc;
+  const bool live = !(s > 1.0);
+  double sn, cs;
+  sincospi(s, &sn, &cs);
+  const double env = 1.0 + cs;
+  const double denv = -pi * sn / c.rc;
+  R[0] = live ? 1.0 : 0.0;
+  dR[0] = 0.0;
+  R[1] = live ? 0.5 * env : 0.0;
+  dR[1] = live ? 0.5 * denv : 0.0;
+  const double arg = -c.lambda * (s - 1.0);
+  const double em1 = expm1(arg);
+  // e^x = 1 + expm1(x) keeps its last bit while the sum does not cancel
+  const double ex = arg > -0.5 ? 1.0 + em1 : exp(arg);
+  const double x = 1.0 - 2.0 * em1 / c.den;
+  const double dx = 2.0 * c.lambda * ex / (c.den * c.rc);
+  double t0 = 1.0, t1 = x, u0 = 1.0, u1 = 2.0 * x;
+#pragma unroll
+  for (int n = 2; n < NRC; ++n) {
+    const double t2 = 2.0 * x * t1 - t0;
+    R[n] = live ? 0.25 * (1.0 - t2) * env : 0.0;
+    dR[n] = live ? 0.25 * ((1.0 - t2) * denv - (double(n) * u1) * dx * env) : 0.0;
+    t0 = t1;
+    t1 = t2;
+    const double u2 = 2.0 * x * u1 - u0;
+    u0 = u1;
+    u1 = u2;
+  }
+}
+
+// groups whose adjoint blocks are on their way at once
+constexpr int kGmAhead = 4;
+
+// NRC: radial rows compiled (>= p.nr; rows from p.nr on meet a zero adjoint).
+template <int LMAX, int NRC, typename In, typename G>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, LMAX >= 6 ? 1 : 2))) void
+density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, int64_t waves) {
+  constexpr int LW = (LMAX + 1) * (LMAX + 1);
+  constexpr int CT = (LW + 15) / 16;
+  constexpr int KS = (NRC + 3) / 4;        // k-steps of four
+  constexpr int YP = LW | 1;               // odd: rows of consecutive edges start in different banks
+  __shared__ double At[2 * NRC][kGmPitch];  // R rows, then R' rows
+  __shared__ double Yt[64][YP];            // Y, then t
+  __shared__ double Al[64];
+  __shared__ int4 gt[64];                  // groups: block, first column, size
+  const int lane = threadIdx.x;
+  const int kq = lane >> 4, cc = lane & 15;
+  const uint64_t lt = (uint64_t(1) << lane) - 1;
+  const int64_t a_begin = int64_t(blockIdx.x) * p.N / waves;
+  const int64_t a_end = (int64_t(blockIdx.x) + 1) * p.N / waves;
+  if (a_begin >= a_end) return;
+  const int64_t block = int64_t(p.nr) * LW;
+  const unsigned voff = unsigned(kq * LW + cc) * unsigned(sizeof(G));
+  auto channel = [&](const GmEdge<In>& edge) {
+    if (!p.species) return 0;
+    return p.species[gm_clamp(edge.j, p.N)];
+  };
+  // Groups of a chunk: each edge's column, and the list of groups.
+  auto group = [&](const GmChunk& c, int kind, int& col, int& ng) {
+    const bool valid = lane < c.cnt;
+    const int sp = kind < 0 ? 0 : (kind >= p.C ? p.C - 1 : kind);
+    int la = 0;
+    for (int j = 0; j < c.na; ++j) la += lane >= __builtin_amdgcn_readlane(c.end, j) ? 1 : 0;
+    col = lane;
+    ng = 0;
+    int base = 0;
+    uint64_t left = gm_ballot(valid);
+    while (left != 0) {
+      const int f = __builtin_ctzll(left);
+      const int fa = __builtin_amdgcn_readlane(la, f);
+      const int fs = __builtin_amdgcn_readlane(sp, f);
+      const bool in = valid && la == fa && sp == fs;
+      const uint64_t m = gm_ballot(in);
+      const int n = __builtin_popcountll(m);
+      if (in) col = base + __builtin_popcountll(m & lt);
+      if (lane == f) gt[ng] = int4{fa * p.C + fs, base, n, 0};
+      ++ng;
+      base += n;
+      left &= ~m;
+    }
+    gm_wave_sync();
+  };
+  auto entry = [&](int k) {
+    const int4 v = gt[k];
+    return int3{__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y),
+                __builtin_amdgcn_readfirstlane(v.z)};
+  };
+  // The adjoint block of a group in the B-operand layout; rows past it read
+  // zero, components past a row are not used.  Without a group the loads are
+  // made all the same, over no bytes, so that the number of loads in flight is
+  // known where the older ones are waited for.
+  auto fetch = [&](int64_t a, bool any, const int3& g, G (&b)[KS][CT]) {
+    const G* src = p.gA + (a * p.C + (any ? g.x : 0)) * block;
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<G*>(src), (short)0, any ? int(block * int64_t(sizeof(G))) : 0, 0x00020000);
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) b[s][ct] = gm_load<G>(rb, voff, unsigned(4 * s * LW + 16 * ct) * sizeof(G));
+  };
+  // t and a of a group's edges
+  auto product = [&](const int3& g, const G (&b)[KS][CT]) {
+    const int pos = g.y, c = g.z;
+#pragma unroll 1
+    for (int m = 0; m < c; m += 4) {
+      const int i = m + (lane & 3);
+      const int ci = pos + (i < c ? i : c - 1);
+      double t[CT], u[CT];
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) t[ct] = u[ct] = 0.0;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const int n = 4 * s + kq < NRC ? 4 * s + kq : NRC - 1;
+        const double ar = At[n][ci], ad = At[NRC + n][ci];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+          t[ct] = __builtin_amdgcn_mfma_f64_4x4x4f64(ar, double(b[s][ct]), t[ct], 0, 0, 0);
+          u[ct] = __builtin_amdgcn_mfma_f64_4x4x4f64(ad, double(b[s][ct]), u[ct], 0, 0, 0);
+        }
+      }
+      const int q = m + kq;
+      const int ce = pos + (q < c ? q : c - 1);
+      double part = 0.0;
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+        if (16 * ct + 15 < LW || 16 * ct + cc < LW) part += u[ct] * Yt[ce][16 * ct + cc];
+      part = gm_sum16(part);
+      if (q < c) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+          if (16 * ct + 15 < LW || 16 * ct + cc < LW) Yt[ce][16 * ct + cc] = t[ct];
+        if (cc == 0) Al[ce] = part;
+      }
+    }
+  };
+
+  // Software pipeline.  Loads return in order, so each is issued before those
+  // that are waited for after it: behind the products of chunk i come the edges
+  // of chunk i + 2 and the offsets after it, and last the first blocks of
+  // chunk i + 1, which then have the chain of chunk i and the basis of chunk
+  // i + 1 to arrive in.  The species of chunk i + 1 are gathered during the
+  // basis and products of chunk i.
+  int64_t e0 = p.row_offsets[a_begin];
+  e0 = gm_clamp(e0, p.E + 1);
+  GmChunk cur = gm_form(a_begin, e0, a_end, gm_window(p, a_begin, a_end, lane), p.E, lane);
+  GmEdge<In> E = gm_edge(p, cur, lane);
+  GmChunk nxt = gm_form(cur.a + cur.na, cur.e + cur.cnt, a_end, gm_window(p, cur.a + cur.na, a_end, lane), p.E, lane);
+  GmEdge<In> NE = gm_edge(p, nxt, lane);
+  int64_t window = gm_window(p, nxt.a + nxt.na, a_end, lane);
+  int col = 0, ng = 0;
+  int3 g[kGmAhead];
+  G b[kGmAhead][KS][CT];
+  group(cur, channel(E), col, ng);
+#pragma unroll
+  for (int d = 0; d < kGmAhead; ++d) {
+    g[d] = entry(d);
+    fetch(cur.a, d < ng, g[d], b[d]);
+  }
+  while (cur.a < a_end) {
+    const bool valid = lane < cur.cnt;
+    const int nsp = channel(NE);
+    const double vx = double(E.x), vy = double(E.y), vz = double(E.z);
+    const double r = d_sqrt(vx * vx + vy * vy + vz * vz);
+    const double sr = r > p.eps ? r : p.eps;
+    const double ux = vx / sr, uy = vy / sr, uz = vz / sr;
+    // ---- basis
+    {
+      double R[NRC], dR[NRC];
+      gm_radial<NRC>(r, radial, R, dR);
+      if (valid) {
+#pragma unroll
+        for (int n = 0; n < NRC; ++n) {
+          At[n][col] = R[n];
+          At[NRC + n][col] = dR[n];
+        }
+      }
+    }
+    if (valid) gm_values<LMAX>(ux, uy, uz, p.nt, Yt[col]);
+    gm_wave_sync();
+
+    // ---- products, group by group
+    for (int k = 0; k < ng; k += kGmAhead) {
+#pragma unroll
+      for (int d = 0; d < kGmAhead; ++d) {
+        if (k + d >= ng) break;
+        product(g[d], b[d]);
+        if (k + d + kGmAhead < ng) {
+          g[d] = entry(k + d + kGmAhead);
+          fetch(cur.a, true, g[d], b[d]);
+        }
+      }
+    }
+    gm_wave_sync();
+
+    // ---- the chunk after next, and the next one's groups and first blocks
+    const int tcol = col;
+    group(nxt, nsp, col, ng);
+    const GmChunk nn = gm_form(nxt.a + nxt.na, nxt.e + nxt.cnt, a_end, window, p.E, lane);
+    const GmEdge<In> NNE = gm_edge(p, nn, lane);
+    window = gm_window(p, nn.a + nn.na, a_end, lane);
+#pragma unroll
+    for (int d = 0; d < kGmAhead; ++d) {
+      g[d] = entry(d);
+      fetch(nxt.a, d < ng, g[d], b[d]);
+    }
+
+    // ---- chain: the contracted gradient of the harmonics
+    if (valid) {
+      double gx, gy, gz;
+      gm_gradient<LMAX>(ux, uy, uz, p.nt, Yt[tcol], gx, gy, gz);
+      const double a = Al[tcol];
+      if (r > p.eps) {  // J^T G with J = (I - u u^T) / r
+        const double ug = ux * gx + uy * gy + uz * gz;
+        gx -= ux * ug;
+        gy -= uy * ug;
+        gz -= uz * ug;
+      }  // else u = v / eps: J = I / eps
+      const int64_t e = cur.e + lane;
+      p.out[3 * e] = In(a * ux + gx / sr);
+      p.out[3 * e + 1] = In(a * uy + gy / sr);
+      p.out[3 * e + 2] = In(a * uz + gz / sr);
+    }
+    gm_wave_sync();  // the tile is read before the next chunk writes it
+    cur = nxt;
+    E = NE;
+    nxt = nn;
+    NE = NNE;
+  }
+}
+
+template <int LMAX, int NRC, typename In, typename G>
+int launch_shape(const GradParams<In, G>& p, hipStream_t s) {
+  auto* const kernel = &density_edge_gradient_mfma_kernel<LMAX, NRC, In, G>;
+  int dev = 0, cus = 0, per_cu = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel),
+                                                   64, 0) != hipSuccess ||
+      per_cu <= 0)
+    per_cu = 4;
+  GmRadial radial;
+  radial.rc = p.cutoff > 2.220446049250313e-16 ? p.cutoff : 2.220446049250313e-16;
+  radial.lambda = p.lambda;
+  radial.den = std::expm1(p.lambda);
+  int64_t waves = int64_t(cus) * per_cu;  // as many as the device holds at once
+  if (waves > p.N) waves = p.N;
+  hipLaunchKernelGGL((density_edge_gradient_mfma_kernel<LMAX, NRC, In, G>), dim3(unsigned(waves)),
+                     dim3(64), 0, s, p, radial, waves);
+  return check_launch("density_edge_gradient_mfma_kernel");
+}
+
+template <int LMAX, typename In, typename G>
+int launch_lmax(const GradParams<In, G>& p, hipStream_t s) {
+  if (p.nr <= 9) return launch_shape<LMAX, 9>(p, s);
+  if (p.nr <= 11) return launch_shape<LMAX, 11>(p, s);
+  if (p.nr <= 13) return launch_shape<LMAX, 13>(p, s);
+  return launch_shape<LMAX, 16>(p, s);
+}
+
+}  // namespace
+
+// Taken where a group fills its four rows on average and the launch fills the
+// chip.  Both sides measured (lane-per-edge / here, us): at 20 000 atoms x 32,
+// l_max 4, n_max 8, ten edges a group 110 / 84 and four 137 / 135; l_max 6,
+// n_max 12, 282 / 158 and 330 / 257; below four edges a group (5 000 x 16,
+// 8 species, l_max 4) 28 / 35; below l_max 4 the blocks are small enough for
+// the lane-per-edge kernel (l_max 2: 33 / 71; l_max 3: 62 / 51 to 111 / 116).
+template <typename In, typename G>
+int launch_edge_gradient_mfma(const GradParams<In, G>& p, int lmax, hipStream_t s) {
+  if (p.mix || p.feats || p.C > (1 << 24)) return YE3T_EUNSUPPORTED;  // a group's block is 32-bit within its chunk
+  if (p.E < 65536 || p.E / 4 < p.N * int64_t(p.C)) return YE3T_EUNSUPPORTED;
+  switch (lmax) {
+    case 4: return launch_lmax<4>(p, s);
+    case 5: return launch_lmax<5>(p, s);
+    case 6: return launch_lmax<6>(p, s);
+    default: return YE3T_EUNSUPPORTED;
+  }
+}
+
+template int launch_edge_gradient_mfma<double, double>(const GradParams<double, double>&, int, hipStream_t);
+template int launch_edge_gradient_mfma<float, float>(const GradParams<float, float>&, int, hipStream_t);
+template int launch_edge_gradient_mfma<float, double>(const GradParams<float, double>&, int, hipStream_t);
+
+}  // namespace ye3t
