@@ -50,28 +50,91 @@ const NormTable& norm_table() {
 }
 
 // ---------------------------------------------------------------------------
-// Radial table: one thread per edge, one Chebyshev pass over n.
-template <typename Real>
-__global__ __launch_bounds__(256) void radial_table_kernel(const Real* __restrict__ radii,
-                                                           const Real* __restrict__ cutoffs,
-                                                           const Real* __restrict__ lambdas, int64_t E,
-                                                           int n_max, Real* __restrict__ values,
-                                                           Real* __restrict__ derivs) {
-  // The basis is evaluated in fp64 for both storage types: the Chebyshev
-  // recurrence amplifies rounding of the warped variable by ~n^2.
-  double v[16], d[16];
-  for (int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; e < E; e += int64_t(gridDim.x) * blockDim.x) {
-    if (derivs) {
-      cheb_exp_cos_row<double, true>(double(radii[e]), double(cutoffs[e]), double(lambdas[e]), n_max, v, d);
-      for (int n = 0; n <= n_max; ++n) {
-        values[e * (n_max + 1) + n] = Real(v[n]);
-        derivs[e * (n_max + 1) + n] = Real(d[n]);
+// ---------------------------------------------------------------------------
+// The per-edge tables.  An edge's row is 25 to 200 values, so a lane that
+// stores its own row puts 64 lines under every store; both kernels write their
+// rows to an LDS tile instead and copy the tile out, which is contiguous in the
+// table, 16 bytes a lane.  Bound by those writes: 640 000 edges with n_max 10,
+// l_max 4 and gradients in fp64 are 640 MB.  Kernel trace there: radial
+// 78 -> 28 us, harmonics 519 -> 94 us (lane-wise stores, the harmonics' recurrences in
+// 1.5 KB of scratch a lane).
+
+// Copies a tile of `rows` x W values (row pitch P in LDS) to `out`: 16 bytes a
+// lane, single values where `out` is not aligned for that and past the last
+// whole vector.
+template <int W, int P, typename Real>
+__device__ inline void copy_rows(const Real* __restrict__ tile, int rows, Real* __restrict__ out) {
+  constexpr int V = 16 / int(sizeof(Real));
+  typedef Real vec __attribute__((ext_vector_type(V)));
+  const int n = rows * W;
+  int done = 0;
+  if (reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+    done = n / V * V;
+    for (int i = int(threadIdx.x) * V; i < done; i += int(blockDim.x) * V) {
+      vec v;
+#pragma unroll
+      for (int q = 0; q < V; ++q) {
+        const unsigned r = unsigned(i + q) / unsigned(W);
+        v[q] = tile[r * P + (unsigned(i + q) - r * W)];
       }
-    } else {
-      cheb_exp_cos_row<double, false>(double(radii[e]), double(cutoffs[e]), double(lambdas[e]), n_max, v, d);
-      for (int n = 0; n <= n_max; ++n) values[e * (n_max + 1) + n] = Real(v[n]);
+      *reinterpret_cast<vec*>(out + i) = v;
     }
   }
+  for (int i = done + int(threadIdx.x); i < n; i += int(blockDim.x)) {
+    const unsigned r = unsigned(i) / unsigned(W);
+    out[i] = tile[r * P + (unsigned(i) - r * W)];
+  }
+}
+
+// Radial table: lane = edge, one Chebyshev pass over n.  128 edges a
+// workgroup: 32 KB of tile at 16 fp64 values and derivatives, five workgroups
+// in a compute unit.
+constexpr int kRadialRows = 128;
+
+template <int NR, bool DERIVS, typename Real>
+__global__ __launch_bounds__(kRadialRows) void radial_table_kernel(const Real* __restrict__ radii,
+                                                                   const Real* __restrict__ cutoffs,
+                                                                   const Real* __restrict__ lambdas, int64_t E,
+                                                                   Real* __restrict__ values,
+                                                                   Real* __restrict__ derivs) {
+  constexpr int P = NR | 1;  // odd: consecutive rows start in different banks
+  __shared__ Real vt[kRadialRows * P];
+  __shared__ Real dt[DERIVS ? kRadialRows * P : 1];
+  const int64_t e0 = int64_t(blockIdx.x) * kRadialRows;
+  const int rows = E - e0 < kRadialRows ? int(E - e0) : kRadialRows;
+  const int t = threadIdx.x;
+  if (t < rows) {
+    // The basis is evaluated in fp64 for both storage types: the Chebyshev
+    // recurrence amplifies rounding of the warped variable by ~n^2.
+    double v[NR], d[NR];
+    cheb_exp_cos_row<double, DERIVS>(double(radii[e0 + t]), double(cutoffs[e0 + t]), double(lambdas[e0 + t]), NR - 1,
+                                     v, d);
+#pragma unroll
+    for (int n = 0; n < NR; ++n) {
+      vt[t * P + n] = Real(v[n]);
+      if (DERIVS) dt[t * P + n] = Real(d[n]);
+    }
+  }
+  __syncthreads();
+  copy_rows<NR, P>(vt, rows, values + e0 * NR);
+  if (DERIVS) copy_rows<NR, P>(dt, rows, derivs + e0 * NR);
+}
+
+template <int NR, typename Real>
+int launch_radial(int nr, const Real* radii, const Real* cutoffs, const Real* lambdas, int64_t E, Real* values,
+                  Real* derivs, hipStream_t s) {
+  if constexpr (NR < 16) {
+    if (nr > NR) return launch_radial<NR + 1>(nr, radii, cutoffs, lambdas, E, values, derivs, s);
+  }
+  const dim3 grid{unsigned((E + kRadialRows - 1) / kRadialRows)};
+  if (derivs) {
+    hipLaunchKernelGGL((radial_table_kernel<NR, true, Real>), grid, dim3(kRadialRows), 0, s, radii, cutoffs, lambdas, E,
+                       values, derivs);
+  } else {
+    hipLaunchKernelGGL((radial_table_kernel<NR, false, Real>), grid, dim3(kRadialRows), 0, s, radii, cutoffs, lambdas, E,
+                       values, derivs);
+  }
+  return check_launch("radial_table_kernel");
 }
 
 // Scheduled radial-angular edge channels: output (e, k) is
@@ -112,9 +175,147 @@ __global__ __launch_bounds__(256) void scheduled_channels_kernel(
   }
 }
 
-// Real SH table with optional Cartesian gradient.  Gradients w.r.t. the unit
-// vector use d/dz Q_l^m = Q_l^{m+1}, projected with (I - u u^T)/|r|
-// (reference ye3t_runtime_core.cpp:226-286, 808-843).
+// Real SH table with optional Cartesian gradient for a compile-time LMAX: lane
+// = edge of a tile of T, and each of four waves takes the orders m of MASK
+// (about a quarter of the components), all in registers.  The tile holds whole
+// rows, up to 100 KB at l_max 6 in fp64, so it is the four waves on one tile that
+// keep a compute unit busy; above that (l_max 7 and 8 in fp64) a tile has 32
+// edges.  Gradients w.r.t. the unit vector use d/dz Q_l^m = Q_l^{m+1},
+// projected with (I - u u^T) / |r| (reference ye3t_runtime_core.cpp:226-286,
+// 808-843).
+template <int LMAX>
+constexpr unsigned sph_orders(int wave) {
+  return wave == 0 ? 0x02u | (LMAX == 7 ? 0x80u : 0x100u)
+         : wave == 1 ? 0x04u | (LMAX == 5 ? 0x20u : 0x40u)
+         : wave == 2 ? 0x08u | (LMAX <= 5 ? 0x10u : 0x20u)
+                     : 0x01u | (LMAX <= 5 ? 0u : 0x10u) | (LMAX == 8 ? 0x80u : 0u);
+}
+
+template <int LMAX, unsigned MASK, bool GRAD, typename Real>
+__device__ inline void sph_tile_rows(const double (&u)[3], double sr, bool project, const NormTable& nt,
+                                     Real* __restrict__ row, Real* __restrict__ grow) {
+  const double sqrt2 = 1.4142135623730950488016887242096981;
+  double cr = 1.0, ci = 0.0, pr = 1.0, pi = 0.0;  // (x + i y)^m and ^(m-1)
+  double qmm = 1.0;                               // Q_m^m
+  const double inv = 1.0 / sr;
+  // the gradient (gx, gy, gz) w.r.t. u of component k, taken to the vector and stored
+  auto put = [&](int k, double gx, double gy, double gz) {
+    if (project) {
+      const double ug = u[0] * gx + u[1] * gy + u[2] * gz;
+      gx -= u[0] * ug;
+      gy -= u[1] * ug;
+      gz -= u[2] * ug;
+    }
+    // g / sr, the reciprocal's product corrected by its remainder
+    auto over = [&](double g) {
+      const double q = g * inv;
+      return fma(fma(-q, sr, g), inv, q);
+    };
+    grow[3 * k] = Real(over(gx));
+    grow[3 * k + 1] = Real(over(gy));
+    grow[3 * k + 2] = Real(over(gz));
+  };
+#pragma unroll
+  for (int m = 0; m <= LMAX; ++m) {
+    if (m > 0) {
+      qmm *= double(2 * m - 1);
+      pr = cr;
+      pi = ci;
+      const double nr = cr * u[0] - ci * u[1];
+      const double ni = cr * u[1] + ci * u[0];
+      cr = nr;
+      ci = ni;
+    }
+    if (((MASK >> m) & 1) == 0) continue;
+    // q: Q_l^m, d: Q_l^{m+1}, by their recurrences in l
+    const double dmm = qmm * double(2 * m + 1);
+    double q2 = 0.0, q1 = 0.0, d2 = 0.0, d1 = 0.0;
+#pragma unroll
+    for (int l = m; l <= LMAX; ++l) {
+      double q, d = 0.0;
+      if (l == m) {
+        q = qmm;
+      } else if (l == m + 1) {
+        q = double(2 * m + 1) * u[2] * qmm;
+        d = dmm;
+      } else {
+        q = (double(2 * l - 1) * u[2] * q1 - double(l + m - 1) * q2) / double(l - m);
+        d = l == m + 2 ? double(2 * m + 3) * u[2] * dmm
+                       : (double(2 * l - 1) * u[2] * d1 - double(l + m) * d2) / double(l - m - 1);
+      }
+      q2 = q1;
+      q1 = q;
+      d2 = d1;
+      d1 = d;
+      const double n = nt.v[l * (kMaxL + 1) + m];
+      const int base = l * l + l;
+      if (m == 0) {
+        row[base] = Real(n * q);
+        if (GRAD) put(base, 0.0, 0.0, n * d);
+      } else {
+        const double s = sqrt2 * n;
+        row[base + m] = Real(s * q * cr);
+        row[base - m] = Real(-s * q * ci);
+        if (GRAD) {
+          const double mq = s * q * double(m), sd = s * d;
+          put(base + m, mq * pr, -mq * pi, sd * cr);
+          put(base - m, -mq * pi, -mq * pr, -sd * ci);
+        }
+      }
+    }
+  }
+}
+
+template <int LMAX, bool GRAD, int T, typename Real>
+__global__ __launch_bounds__(256) void sph_tile_kernel(const Real* __restrict__ vec, int64_t E, double eps,
+                                                       NormTable nt, Real* __restrict__ values,
+                                                       Real* __restrict__ grads) {
+  constexpr int W = (LMAX + 1) * (LMAX + 1);
+  constexpr int P = W | 1, GP = 3 * W | 1;  // odd: consecutive rows start in different banks
+  __shared__ Real vt[T * P];
+  __shared__ Real gt[GRAD ? T * GP : 1];
+  const int64_t e0 = int64_t(blockIdx.x) * T;
+  const int rows = E - e0 < T ? int(E - e0) : T;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (lane < rows) {
+    const int64_t e = e0 + lane;
+    const double x0 = double(vec[3 * e]), y0 = double(vec[3 * e + 1]), z0 = double(vec[3 * e + 2]);
+    const double r = d_sqrt(x0 * x0 + y0 * y0 + z0 * z0);
+    const double sr = r > eps ? r : eps;
+    const double u[3] = {x0 / sr, y0 / sr, z0 / sr};
+    Real* const row = vt + lane * P;
+    Real* const grow = gt + (GRAD ? lane * GP : 0);
+    const bool project = r > eps;
+    if (wave == 0) sph_tile_rows<LMAX, sph_orders<LMAX>(0), GRAD>(u, sr, project, nt, row, grow);
+    else if (wave == 1) sph_tile_rows<LMAX, sph_orders<LMAX>(1), GRAD>(u, sr, project, nt, row, grow);
+    else if (wave == 2) sph_tile_rows<LMAX, sph_orders<LMAX>(2), GRAD>(u, sr, project, nt, row, grow);
+    else sph_tile_rows<LMAX, sph_orders<LMAX>(3), GRAD>(u, sr, project, nt, row, grow);
+  }
+  __syncthreads();
+  copy_rows<W, P>(vt, rows, values + e0 * W);
+  if (GRAD) copy_rows<3 * W, GP>(gt, rows, grads + e0 * 3 * W);
+}
+
+template <int LMAX, typename Real>
+int launch_sph_tile(int lmax, const Real* vec, int64_t E, double eps, Real* values, Real* grads, hipStream_t s) {
+  if constexpr (LMAX < 8) {
+    if (lmax > LMAX) return launch_sph_tile<LMAX + 1>(lmax, vec, E, eps, values, grads, s);
+  }
+  constexpr int T = LMAX > 6 && sizeof(Real) == 8 ? 32 : 64;
+  const dim3 grid{unsigned((E + T - 1) / T)};
+  if (grads) {
+    hipLaunchKernelGGL((sph_tile_kernel<LMAX, true, T, Real>), grid, dim3(256), 0, s, vec, E, eps, norm_table(), values,
+                       grads);
+  } else {
+    hipLaunchKernelGGL((sph_tile_kernel<LMAX, false, T, Real>), grid, dim3(256), 0, s, vec, E, eps, norm_table(),
+                       values, grads);
+  }
+  return check_launch("sph_tile_kernel");
+}
+
+// The same table for any l_max (l_max 9 and above): one lane per edge, the
+// recurrences in scratch.
 template <typename Real>
 __global__ __launch_bounds__(128) void real_sph_table_kernel(const Real* __restrict__ vec, int64_t E, int lmax,
                                                              double eps, NormTable nt, Real* __restrict__ values,
@@ -360,19 +561,14 @@ int ye3t_hip_radial_table(int dtype, const void* radii, const void* cutoffs, con
   YE3T_REQUIRE(n_max >= 0 && n_max < 16, "max_radial_index must be in [0, 15], got %lld", (long long)n_max);
   if (E == 0) return YE3T_OK;
   YE3T_REQUIRE(radii && cutoffs && lambdas && values, "NULL input or output");
-  const unsigned grid = grid_for(E, 256);
-  if (dtype == YE3T_F64) {
-    hipLaunchKernelGGL(radial_table_kernel<double>, dim3(grid), dim3(256), 0, as_stream(stream),
-                       (const double*)radii, (const double*)cutoffs, (const double*)lambdas, E, int(n_max),
-                       (double*)values, (double*)derivs);
-  } else if (dtype == YE3T_F32) {
-    hipLaunchKernelGGL(radial_table_kernel<float>, dim3(grid), dim3(256), 0, as_stream(stream),
-                       (const float*)radii, (const float*)cutoffs, (const float*)lambdas, E, int(n_max),
-                       (float*)values, (float*)derivs);
-  } else {
-    return set_error(YE3T_EDTYPE, "unsupported dtype %d", dtype);
-  }
-  return check_launch("radial_table_kernel");
+  YE3T_REQUIRE((E + kRadialRows - 1) / kRadialRows <= INT32_MAX, "too many edges for one launch");
+  if (dtype == YE3T_F64)
+    return launch_radial<1>(int(n_max) + 1, (const double*)radii, (const double*)cutoffs, (const double*)lambdas, E,
+                            (double*)values, (double*)derivs, as_stream(stream));
+  if (dtype == YE3T_F32)
+    return launch_radial<1>(int(n_max) + 1, (const float*)radii, (const float*)cutoffs, (const float*)lambdas, E,
+                            (float*)values, (float*)derivs, as_stream(stream));
+  return set_error(YE3T_EDTYPE, "unsupported dtype %d", dtype);
 }
 
 int ye3t_hip_scheduled_radial_angular_channels(int dtype, int64_t edge_count, int64_t radial_width,
@@ -421,6 +617,12 @@ int ye3t_hip_real_sph_table(int dtype, const void* vec, int64_t E, int64_t lmax,
   YE3T_REQUIRE(lmax >= 0 && lmax <= kMaxL, "maximum_angular_momentum must be in [0, %d]", kMaxL);
   if (E == 0) return YE3T_OK;
   YE3T_REQUIRE(vec && values, "NULL input or output");
+  if (lmax <= 8 && E <= int64_t(INT32_MAX) * 32) {
+    if (dtype == YE3T_F64)
+      return launch_sph_tile<0>(int(lmax), (const double*)vec, E, eps, (double*)values, (double*)grads, as_stream(stream));
+    if (dtype == YE3T_F32)
+      return launch_sph_tile<0>(int(lmax), (const float*)vec, E, eps, (float*)values, (float*)grads, as_stream(stream));
+  }
   const unsigned grid = grid_for(E, 128);
   if (dtype == YE3T_F64) {
     hipLaunchKernelGGL(real_sph_table_kernel<double>, dim3(grid), dim3(128), 0, as_stream(stream),

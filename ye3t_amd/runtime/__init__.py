@@ -82,9 +82,13 @@ def _radial_operands(radii, cutoffs, lambdas, name):
 
     radii = torch.as_tensor(radii)
     _require_device(radii, name)
-    cutoffs = torch.as_tensor(cutoffs, dtype=radii.dtype, device=radii.device).expand_as(radii).contiguous()
-    lambdas = torch.as_tensor(lambdas, dtype=radii.dtype, device=radii.device).expand_as(radii).contiguous()
-    return radii.contiguous(), cutoffs, lambdas
+
+    def operand(v):
+        if isinstance(v, (int, float)):  # filled on the device: a copy of one number would be waited for
+            return torch.full(radii.shape, v, dtype=radii.dtype, device=radii.device)
+        return torch.as_tensor(v, dtype=radii.dtype, device=radii.device).expand_as(radii).contiguous()
+
+    return radii.contiguous(), operand(cutoffs), operand(lambdas)
 
 
 def cheb_exp_cos_radial_table_with_derivative(radii, cutoffs, lambdas, maximum_radial_index, backend="auto"):
