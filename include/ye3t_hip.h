@@ -127,21 +127,29 @@ int ye3t_hip_density_accumulate_adjoint(int dtype, const void* atomic_adjoint, c
                                         int64_t edge_count, int64_t channel_count, int64_t atom_count,
                                         void* edge_adjoint, ye3t_stream_t stream);
 
-/* Checks index inputs on the device in one pass and waits for the answer.
- * row_offsets (NULL: not checked) has atom_count + 1 entries, indices (NULL:
- * not checked) index_count entries to lie in [0, index_limit), species (NULL:
- * not checked) atom_count entries to lie in [0, species_count).  result (host,
- * YE3T_CHECK_RESULTS words) receives: [0] row_offsets[0]; [1]
- * row_offsets[atom_count]; then 1 for each fault, else 0: [2] row_offsets fall
- * somewhere, [3] an index is out of range, [4] a species is out of range, [5]
- * without row_offsets, the indices fall somewhere.  Synchronises `stream`;
+/* Checks index arrays on the device in one pass and waits for the answer.
+ * Each of the check_count (at most YE3T_MAX_CHECKS) arrays receives four words
+ * of result (host, 4 * check_count): its first and last value, 1 if a value is
+ * outside [first, limit), and, where `ordered`, 1 if a value is below its
+ * predecessor.  An empty array's words are zero.  Synchronises `stream`;
  * YE3T_EUNSUPPORTED, with nothing launched, while the stream is captured.
  * Replaces the host guards in front of the reference's gathers
  * (execution_plan_cuda.cu:37-197). */
-#define YE3T_CHECK_RESULTS 6
-int ye3t_hip_check_indices(const int64_t* row_offsets, int64_t atom_count, const int64_t* indices,
-                           int64_t index_count, int64_t index_limit, const int32_t* species, int64_t species_count,
-                           int64_t* result, ye3t_stream_t stream);
+#define YE3T_MAX_CHECKS 4
+typedef struct {
+  const void* data; /* device */
+  int64_t count;
+  int64_t first, limit;
+  int width; /* bytes of a value: 4 or 8, signed */
+  int ordered;
+} ye3t_index_check;
+int ye3t_hip_check_indices(const ye3t_index_check* checks, int check_count, int64_t* result, ye3t_stream_t stream);
+
+/* row_offsets[i] = number of edges with a centre below i, for i <= atom_count,
+ * of centres that do not fall and lie in [0, atom_count) (checked by the
+ * caller). */
+int ye3t_hip_csr_offsets(const int64_t* centers, int64_t edge_count, int64_t atom_count, int64_t* row_offsets,
+                         ye3t_stream_t stream);
 
 /* Fused stage 1: A[i, c, r, lm] = sum_{e in row i} w_c(e) R_r(|v_e|) Y_lm(v_e/|v_e|).
  * One pass over edges: radial basis and real SH in registers, per-atom CSR

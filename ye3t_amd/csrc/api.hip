@@ -50,6 +50,15 @@ const NormTable& norm_table() {
 }
 
 // ---------------------------------------------------------------------------
+inline unsigned grid_for(int64_t work, int threads) {
+  int64_t g = (work + threads - 1) / threads;
+  if (g < 1) g = 1;
+  if (g > (1 << 20)) g = 1 << 20;
+  return unsigned(g);
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 // ---------------------------------------------------------------------------
 // The per-edge tables.  An edge's row is 25 to 200 values, so a lane that
 // stores its own row puts 64 lines under every store; both kernels write their
@@ -140,39 +149,150 @@ int launch_radial(int nr, const Real* radii, const Real* cutoffs, const Real* la
 // Scheduled radial-angular edge channels: output (e, k) is
 // scale_k R[e, ri_k] Y[e, ai_k] when channel k takes every edge type
 // (type -1) or edge e's type, zero otherwise, with its Cartesian derivative
-// scale_k (dR[e, ri_k] dir[e] Y[e, ai_k] + R[e, ri_k] dY[e, ai_k]).  One thread
-// per output.  The products are rounded in the reference core's order
+// scale_k (dR[e, ri_k] dir[e] Y[e, ai_k] + R[e, ri_k] dY[e, ai_k]).  The
+// products are rounded in the reference core's order
 // (ye3t_runtime_core.cpp:1550-1604) with no fused multiply-adds, so the
 // results are the core's bit for bit.  Indices are validated by the caller;
 // the kernel clamps them into the tables rather than faulting.
+//
+// Four values are written for each of E K outputs; those writes bound it.  A
+// workgroup takes whole edges, about 4 096 outputs, with their table rows and the
+// schedule in LDS (an output reads ten values, each of them shared by a row of
+// others) and lane = output; the three components of a wave's 64 outputs go
+// through LDS too, so that every store is contiguous.  240 000 edges x 144
+// channels in fp64 (1.1 GB written): 425 -> 250 us (one thread an output with
+// a 64-bit division and 24-byte strided stores before; 354 us with the rows
+// read from memory).
+constexpr int kChannelThreads = 256;
+constexpr int64_t kChannelTable = 1024;     // channels whose schedule is held in LDS (24 KB)
+constexpr int64_t kChannelRows = 32 * 1024;  // bytes of edge rows held in LDS
+
 template <typename Real>
-__global__ __launch_bounds__(256) void scheduled_channels_kernel(
+struct ChannelSchedule {
+  int64_t type;
+  Real scale;
+  int32_t ri, ai;
+};
+
+// HELD: the schedule and the edges' rows are in LDS.
+template <bool HELD, typename Real>
+__global__ __launch_bounds__(kChannelThreads) void scheduled_channels_kernel(
     const Real* __restrict__ rv, const Real* __restrict__ rd, const Real* __restrict__ av,
     const Real* __restrict__ ad, const Real* __restrict__ dir, const int64_t* __restrict__ edge_types,
     const int64_t* __restrict__ cri, const int64_t* __restrict__ cai, const int64_t* __restrict__ ctype,
-    const Real* __restrict__ cscale, int64_t E, int64_t NR, int64_t NA, int64_t K, Real* __restrict__ values,
-    Real* __restrict__ derivs) {
+    const Real* __restrict__ cscale, int64_t E, int64_t NR, int64_t NA, int64_t K, int64_t tile,
+    Real* __restrict__ values, Real* __restrict__ derivs) {
 #pragma clang fp contract(off)
-  const int64_t total = E * K;
-  for (int64_t o = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; o < total; o += int64_t(gridDim.x) * blockDim.x) {
-    const int64_t e = o / K, k = o - e * K;
-    const int64_t t = ctype[k];
-    Real* const d = derivs + 3 * o;
-    if (t >= 0 && edge_types[e] != t) {
-      values[o] = Real(0);
-      d[0] = d[1] = d[2] = Real(0);
-      continue;
-    }
-    int64_t ri = cri[k], ai = cai[k];
-    ri = ri < 0 ? 0 : (ri >= NR ? NR - 1 : ri);
-    ai = ai < 0 ? 0 : (ai >= NA ? NA - 1 : ai);
-    const Real r = rv[e * NR + ri], a = av[e * NA + ai], sc = cscale[k];
-    const Real dr = rd[e * NR + ri];
-    values[o] = sc * r * a;
-    const Real* const ya = ad + 3 * (e * NA + ai);
-    const Real* const u = dir + 3 * e;
-    for (int x = 0; x < 3; ++x) d[x] = sc * (dr * u[x] * a + r * ya[x]);
+  constexpr int V = 16 / int(sizeof(Real));
+  typedef Real vec __attribute__((ext_vector_type(V)));
+  extern __shared__ __align__(16) unsigned char channel_smem[];
+  __shared__ __align__(16) Real stage[kChannelThreads / 64][192];
+  auto schedule = [&](int64_t k) {
+    ChannelSchedule<Real> c;
+    const int64_t ri = cri[k], ai = cai[k];
+    c.type = ctype[k];
+    c.scale = cscale[k];
+    c.ri = int32_t(ri < 0 ? 0 : (ri >= NR ? NR - 1 : ri));
+    c.ai = int32_t(ai < 0 ? 0 : (ai >= NA ? NA - 1 : ai));
+    return c;
+  };
+  const int64_t e0 = int64_t(blockIdx.x) * tile;
+  const int64_t edges = E - e0 < tile ? E - e0 : tile;
+  ChannelSchedule<Real>* const table = reinterpret_cast<ChannelSchedule<Real>*>(channel_smem);
+  int64_t* const type = reinterpret_cast<int64_t*>(table + (HELD ? K : 0));
+  Real* const srv = reinterpret_cast<Real*>(type + (HELD ? tile : 0));
+  Real* const srd = srv + (HELD ? tile * NR : 0);
+  Real* const sav = srd + (HELD ? tile * NR : 0);
+  Real* const sad = sav + (HELD ? tile * NA : 0);
+  Real* const sdir = sad + (HELD ? tile * NA * 3 : 0);
+  if (HELD) {
+    auto hold = [&](Real* to, const Real* from, int64_t n) {
+      for (int64_t i = threadIdx.x; i < n; i += kChannelThreads) to[i] = from[i];
+    };
+    for (int64_t k = threadIdx.x; k < K; k += kChannelThreads) table[k] = schedule(k);
+    for (int64_t i = threadIdx.x; i < edges; i += kChannelThreads) type[i] = edge_types[e0 + i];
+    hold(srv, rv + e0 * NR, edges * NR);
+    hold(srd, rd + e0 * NR, edges * NR);
+    hold(sav, av + e0 * NA, edges * NA);
+    hold(sad, ad + e0 * NA * 3, edges * NA * 3);
+    hold(sdir, dir + e0 * 3, edges * 3);
+    __syncthreads();
   }
+  const int64_t outputs = edges * K;
+  const int64_t o0 = e0 * K;
+  const int lane = threadIdx.x & 63;
+  Real* const mine = stage[threadIdx.x >> 6];
+  const bool aligned = reinterpret_cast<uintptr_t>(derivs + 3 * o0) % 16 == 0;
+  // the lane's channel and edge (of the tile) advance by 256 outputs a step
+  const int dk = int(kChannelThreads % K), de = int(kChannelThreads / K);
+  int64_t e = int64_t(threadIdx.x) / K, k = int64_t(threadIdx.x) % K;
+  for (int64_t w = threadIdx.x - lane; w < outputs; w += kChannelThreads) {
+    const int left = outputs - w < 64 ? int(outputs - w) : 64;  // outputs of this wave's step
+    if (lane < left) {
+      const ChannelSchedule<Real> c = HELD ? table[k] : schedule(k);
+      Real v = Real(0), d0 = Real(0), d1 = Real(0), d2 = Real(0);
+      if (!(c.type >= 0 && (HELD ? type[e] : edge_types[e0 + e]) != c.type)) {
+        const int64_t row = HELD ? e : e0 + e;
+        const Real r = (HELD ? srv : rv)[row * NR + c.ri], dr = (HELD ? srd : rd)[row * NR + c.ri];
+        const Real a = (HELD ? sav : av)[row * NA + c.ai], sc = c.scale;
+        const Real* const ya = (HELD ? sad : ad) + 3 * (row * NA + c.ai);
+        const Real* const u = (HELD ? sdir : dir) + 3 * row;
+        v = sc * r * a;
+        d0 = sc * (dr * u[0] * a + r * ya[0]);
+        d1 = sc * (dr * u[1] * a + r * ya[1]);
+        d2 = sc * (dr * u[2] * a + r * ya[2]);
+      }
+      values[o0 + w + lane] = v;
+      mine[3 * lane] = d0;
+      mine[3 * lane + 1] = d1;
+      mine[3 * lane + 2] = d2;
+    }
+    // the wave's own 192 components: written by its lanes, read by others of them
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    Real* const out = derivs + 3 * (o0 + w);
+    const int n = 3 * left;
+    const int whole = aligned ? n / V * V : 0;
+    for (int i = lane * V; i < whole; i += 64 * V)
+      *reinterpret_cast<vec*>(out + i) = *reinterpret_cast<const vec*>(mine + i);
+    for (int i = whole + lane; i < n; i += 64) out[i] = mine[i];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    e += de;
+    k += dk;
+    if (k >= K) {
+      k -= K;
+      ++e;
+    }
+  }
+}
+
+template <typename Real>
+int launch_channels(const Real* rv, const Real* rd, const Real* av, const Real* ad, const Real* dir,
+                    const int64_t* types, const int64_t* cri, const int64_t* cai, const int64_t* ctype,
+                    const Real* cscale, int64_t E, int64_t NR, int64_t NA, int64_t K, Real* values, Real* derivs,
+                    hipStream_t s) {
+  // edges of a workgroup: about 4 096 outputs, as far as their rows fit, and an
+  // even number (rows of three fp64 values start on 16 bytes every second output)
+  const int64_t row = (2 * NR + 4 * NA + 3) * int64_t(sizeof(Real)) + 8;
+  const int64_t fit = kChannelRows / row;
+  const bool held = K <= kChannelTable && fit >= 2;
+  int64_t tile = 4096 / K;
+  if (held && tile > fit) tile = fit;
+  tile = tile < 2 ? 2 : tile / 2 * 2;
+  const int64_t groups = (E + tile - 1) / tile;
+  YE3T_REQUIRE(groups <= INT32_MAX, "too many edges for one launch");
+  if (held) {
+    hipLaunchKernelGGL((scheduled_channels_kernel<true, Real>), dim3(unsigned(groups)), dim3(kChannelThreads),
+                       size_t(K) * sizeof(ChannelSchedule<Real>) + size_t(tile * row), s, rv, rd, av, ad, dir, types,
+                       cri, cai, ctype, cscale, E, NR, NA, K, tile, values, derivs);
+  } else {
+    hipLaunchKernelGGL((scheduled_channels_kernel<false, Real>), dim3(unsigned(groups)), dim3(kChannelThreads), 0, s,
+                       rv, rd, av, ad, dir, types, cri, cai, ctype, cscale, E, NR, NA, K, tile, values, derivs);
+  }
+  return check_launch("scheduled_channels_kernel");
 }
 
 // Real SH table with optional Cartesian gradient for a compile-time LMAX: lane
@@ -431,70 +551,94 @@ __global__ __launch_bounds__(256) void density_csr_kernel(const Real* __restrict
   }
 }
 
-// Gather of centre-row adjoints to edge rows.  A workgroup of 256 threads
-// copies whole edge rows: 256 / CV rows at a time when a row is at most 256
-// vectors (V = 16 bytes when the rows allow it), else one row in a loop;
-// indices within the group are 32-bit.  The output is streamed with
-// non-temporal stores (written once, not re-read here).  Centres are validated
-// by the caller; an index outside [0, N) is clamped so that no access leaves
-// the array.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+// Row offsets of centre-sorted edges: lane = row, a bisection for the first
+// edge whose centre is not below it (any run of empty rows costs the same).
+__global__ __launch_bounds__(256) void csr_offsets_kernel(const int64_t* __restrict__ centers, int64_t E, int64_t N,
+                                                          int64_t* __restrict__ offsets) {
+  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i <= N; i += int64_t(gridDim.x) * blockDim.x) {
+    int64_t lo = 0, hi = E;  // centers[lo - 1] < i <= centers[hi]
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (centers[mid] < i) lo = mid + 1;
+      else hi = mid;
+    }
+    offsets[i] = lo;
+  }
+}
+
+// Gather of centre-row adjoints to edge rows.  A workgroup copies 256 vectors
+// at a time (V = 16 bytes when the rows allow it), eight steps over consecutive
+// vectors of the edge rows with every step's read requested before the first
+// write; the output is streamed with non-temporal stores (written once, not
+// re-read here).  Centres are validated by the caller; an index outside [0, N)
+// is clamped so that no access leaves the array.  240 000 edges x 144 channels
+// in fp64 (276 MB written): 92 -> 67 us (one step a workgroup before).
+constexpr int kGatherSteps = 8;
 
 template <typename V>
 __global__ __launch_bounds__(256) void density_adjoint_kernel(const V* __restrict__ adj,
                                                               const int64_t* __restrict__ centers, int64_t E,
-                                                              int CV, int64_t N, V* __restrict__ out) {
-  const int epb = CV >= 256 ? 1 : 256 / CV;  // edge rows per pass of the workgroup
-  const int span = epb * CV;
-  for (int64_t e0 = int64_t(blockIdx.x) * epb; e0 < E; e0 += int64_t(gridDim.x) * epb) {
-    for (int t = threadIdx.x; t < span; t += 256) {
-      const int de = t / CV;
-      const int c = t - de * CV;
-      const int64_t e = e0 + de;
-      if (e < E) {
+                                                              int64_t CV, int64_t N, V* __restrict__ out) {
+  const int64_t total = E * CV;
+  const int64_t dc = 256 % CV, de = 256 / CV;
+  for (int64_t x0 = int64_t(blockIdx.x) * (256 * kGatherSteps); x0 < total;
+       x0 += int64_t(gridDim.x) * (256 * kGatherSteps)) {
+    const int64_t x = x0 + threadIdx.x;
+    int64_t e = x / CV, c = x - e * CV;
+    V v[kGatherSteps];
+#pragma unroll
+    for (int k = 0; k < kGatherSteps; ++k) {
+      if (x + 256 * k < total) {
         int64_t i = centers[e];
         i = i < 0 ? 0 : (i >= N ? N - 1 : i);
-        __builtin_nontemporal_store(adj[i * CV + c], out + e * CV + c);
+        v[k] = adj[i * CV + c];
+      }
+      e += de;
+      c += dc;
+      if (c >= CV) {
+        c -= CV;
+        ++e;
       }
     }
+#pragma unroll
+    for (int k = 0; k < kGatherSteps; ++k)
+      if (x + 256 * k < total) __builtin_nontemporal_store(v[k], out + x + 256 * k);
   }
 }
 
-// Range checks of a density's index inputs in one pass over them: nothing is
-// reduced, a lane that sees a violation stores its word of `status` (host
-// memory the device can write, zeroed by the host), and the first and last
-// offsets are copied there.  A structure of 50 000 atoms and 1.2 M edges is
+// Range checks of index inputs in one pass over them, one grid row an array:
+// nothing is reduced, a lane that sees a violation stores its word of `status`
+// (host memory the device can write, zeroed by the host), and the first and
+// last values are copied there.  A structure of 50 000 atoms and 1.2 M edges is
 // 10 MB, about 4 us of reads; taken as torch reductions with a read-back each
 // (minimum and maximum of the neighbours, first and last offset, monotony) the
 // same checks are six kernels and five synchronisations: a 16-channel density
 // and product of 50 000 atoms took 260 us with those, 169 us with this, and
 // one of 128 atoms 110 and 40 us.
+struct IndexChecks {
+  ye3t_index_check c[YE3T_MAX_CHECKS];
+};
+
 template <typename T>
-__device__ inline void check_range(const T* __restrict__ v, int64_t n, int64_t limit, bool ordered,
-                                   int64_t* __restrict__ bad, int64_t* __restrict__ descends) {
-  const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-  for (int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < n; k += stride) {
+__device__ inline void check_one(const ye3t_index_check& c, int64_t* __restrict__ status) {
+  const T* __restrict__ v = static_cast<const T*>(c.data);
+  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (t == 0) {
+    status[0] = int64_t(v[0]);
+    status[1] = int64_t(v[c.count - 1]);
+  }
+  for (int64_t k = t; k < c.count; k += int64_t(gridDim.x) * blockDim.x) {
     const int64_t x = int64_t(v[k]);
-    if (x < 0 || x >= limit) *bad = 1;
-    if (ordered && k > 0 && int64_t(v[k - 1]) > x) *descends = 1;
+    if (x < c.first || x >= c.limit) status[2] = 1;
+    if (c.ordered && k > 0 && int64_t(v[k - 1]) > x) status[3] = 1;
   }
 }
 
-__global__ __launch_bounds__(256) void check_indices_kernel(const int64_t* __restrict__ offsets, int64_t N,
-                                                            const int64_t* __restrict__ indices, int64_t count,
-                                                            int64_t limit, const int32_t* __restrict__ species,
-                                                            int64_t species_count, int64_t* __restrict__ status) {
-  if (offsets != nullptr) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      status[0] = offsets[0];
-      status[1] = offsets[N];
-    }
-    const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-    for (int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < N; k += stride)
-      if (offsets[k] > offsets[k + 1]) status[2] = 1;
-  }
-  if (indices != nullptr) check_range(indices, count, limit, offsets == nullptr, status + 3, status + 5);
-  if (species != nullptr) check_range(species, N, species_count, false, status + 4, status + 6);
+__global__ __launch_bounds__(256) void check_indices_kernel(IndexChecks checks, int64_t* __restrict__ status) {
+  const ye3t_index_check& c = checks.c[blockIdx.y];
+  if (c.count == 0) return;
+  if (c.width == 8) check_one<int64_t>(c, status + 4 * blockIdx.y);
+  else check_one<int32_t>(c, status + 4 * blockIdx.y);
 }
 
 // The status words of the calling thread: pinned host memory, made at the
@@ -507,14 +651,8 @@ struct CheckStatus {
     if (words != nullptr) (void)hipHostFree(words);
   }
 };
-constexpr int kCheckWords = 8;
+constexpr int kCheckWords = 4 * YE3T_MAX_CHECKS;
 
-inline unsigned grid_for(int64_t work, int threads) {
-  int64_t g = (work + threads - 1) / threads;
-  if (g < 1) g = 1;
-  if (g > (1 << 20)) g = 1 << 20;
-  return unsigned(g);
-}
 
 }  // namespace ye3t
 
@@ -589,25 +727,21 @@ int ye3t_hip_scheduled_radial_angular_channels(int dtype, int64_t edge_count, in
                    edge_types && channel_radial_indices && channel_angular_indices && channel_types &&
                    channel_scales && edge_values && edge_derivatives,
                "NULL input or output");
-  const unsigned grid = grid_for(edge_count * channel_count, 256);
-  if (dtype == YE3T_F64) {
-    hipLaunchKernelGGL(scheduled_channels_kernel<double>, dim3(grid), dim3(256), 0, as_stream(stream),
-                       (const double*)radial_values, (const double*)radial_derivatives,
-                       (const double*)angular_values, (const double*)angular_derivatives,
-                       (const double*)radial_directions, edge_types, channel_radial_indices,
-                       channel_angular_indices, channel_types, (const double*)channel_scales, edge_count,
-                       radial_width, angular_width, channel_count, (double*)edge_values, (double*)edge_derivatives);
-  } else if (dtype == YE3T_F32) {
-    hipLaunchKernelGGL(scheduled_channels_kernel<float>, dim3(grid), dim3(256), 0, as_stream(stream),
-                       (const float*)radial_values, (const float*)radial_derivatives,
-                       (const float*)angular_values, (const float*)angular_derivatives,
-                       (const float*)radial_directions, edge_types, channel_radial_indices,
-                       channel_angular_indices, channel_types, (const float*)channel_scales, edge_count,
-                       radial_width, angular_width, channel_count, (float*)edge_values, (float*)edge_derivatives);
-  } else {
-    return set_error(YE3T_EDTYPE, "unsupported dtype %d", dtype);
-  }
-  return check_launch("scheduled_channels_kernel");
+  YE3T_REQUIRE(radial_width <= INT32_MAX && angular_width <= INT32_MAX, "tables too wide");
+  if (dtype == YE3T_F64)
+    return launch_channels((const double*)radial_values, (const double*)radial_derivatives,
+                           (const double*)angular_values, (const double*)angular_derivatives,
+                           (const double*)radial_directions, edge_types, channel_radial_indices,
+                           channel_angular_indices, channel_types, (const double*)channel_scales, edge_count,
+                           radial_width, angular_width, channel_count, (double*)edge_values,
+                           (double*)edge_derivatives, as_stream(stream));
+  if (dtype == YE3T_F32)
+    return launch_channels((const float*)radial_values, (const float*)radial_derivatives, (const float*)angular_values,
+                           (const float*)angular_derivatives, (const float*)radial_directions, edge_types,
+                           channel_radial_indices, channel_angular_indices, channel_types,
+                           (const float*)channel_scales, edge_count, radial_width, angular_width, channel_count,
+                           (float*)edge_values, (float*)edge_derivatives, as_stream(stream));
+  return set_error(YE3T_EDTYPE, "unsupported dtype %d", dtype);
 }
 
 int ye3t_hip_real_sph_table(int dtype, const void* vec, int64_t E, int64_t lmax, double eps, void* values,
@@ -655,17 +789,25 @@ int ye3t_hip_density_accumulate_csr(int dtype, const void* ev, const int64_t* of
   return check_launch("density_csr_kernel");
 }
 
-int ye3t_hip_check_indices(const int64_t* row_offsets, int64_t atom_count, const int64_t* indices, int64_t index_count,
-                           int64_t index_limit, const int32_t* species, int64_t species_count, int64_t* result,
-                           ye3t_stream_t stream) {
+int ye3t_hip_check_indices(const ye3t_index_check* checks, int check_count, int64_t* result, ye3t_stream_t stream) {
   clear_error();
-  YE3T_REQUIRE(atom_count >= 0 && index_count >= 0, "negative size");
-  YE3T_REQUIRE(result != nullptr, "NULL result");
+  YE3T_REQUIRE(check_count >= 1 && check_count <= YE3T_MAX_CHECKS, "between 1 and %d checks", YE3T_MAX_CHECKS);
+  YE3T_REQUIRE(checks != nullptr && result != nullptr, "NULL checks or result");
+  IndexChecks all = {};
+  int64_t most = 0;
+  for (int k = 0; k < check_count; ++k) {
+    YE3T_REQUIRE(checks[k].count >= 0 && (checks[k].width == 4 || checks[k].width == 8), "bad index check");
+    YE3T_REQUIRE(checks[k].count == 0 || checks[k].data != nullptr, "NULL indices");
+    all.c[k] = checks[k];
+    if (checks[k].count > most) most = checks[k].count;
+  }
   const hipStream_t s = as_stream(stream);
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   YE3T_CHECK_HIP(hipStreamIsCapturing(s, &capture));
   if (capture != hipStreamCaptureStatusNone)
     return set_error(YE3T_EUNSUPPORTED, "indices cannot be checked while the stream is captured");
+  for (int k = 0; k < 4 * check_count; ++k) result[k] = 0;
+  if (most == 0) return YE3T_OK;
   static thread_local CheckStatus status;
   if (status.words == nullptr) {
     void* words = nullptr;
@@ -673,18 +815,25 @@ int ye3t_hip_check_indices(const int64_t* row_offsets, int64_t atom_count, const
     status.words = static_cast<int64_t*>(words);
   }
   for (int k = 0; k < kCheckWords; ++k) status.words[k] = 0;
-  // eight indices per lane and pass: enough wavefronts to cover the latency of a
-  // short read, and few enough workgroups for the smallest calls to start at once
-  const int64_t most = index_count > atom_count ? index_count : atom_count;
-  const unsigned grid = grid_for((most + 7) / 8, 256);
-  hipLaunchKernelGGL(check_indices_kernel, dim3(grid), dim3(256), 0, s, row_offsets, atom_count,
-                     index_count > 0 ? indices : nullptr, index_count, index_limit,
-                     atom_count > 0 ? species : nullptr, species_count, status.words);
+  // eight indices per lane: enough wavefronts to cover the latency of a short
+  // read, and few enough workgroups for the smallest calls to start at once
+  hipLaunchKernelGGL(check_indices_kernel, dim3(grid_for((most + 7) / 8, 256), unsigned(check_count)), dim3(256), 0, s,
+                     all, status.words);
   const int rc = check_launch("check_indices_kernel");
   if (rc != YE3T_OK) return rc;
   YE3T_CHECK_HIP(hipStreamSynchronize(s));
-  for (int k = 0; k < YE3T_CHECK_RESULTS; ++k) result[k] = status.words[k];
+  for (int k = 0; k < 4 * check_count; ++k) result[k] = status.words[k];
   return YE3T_OK;
+}
+
+int ye3t_hip_csr_offsets(const int64_t* centers, int64_t edge_count, int64_t atom_count, int64_t* row_offsets,
+                         ye3t_stream_t stream) {
+  clear_error();
+  YE3T_REQUIRE(edge_count >= 0 && atom_count >= 0, "negative size");
+  YE3T_REQUIRE(row_offsets != nullptr && (edge_count == 0 || centers != nullptr), "NULL centres or output");
+  hipLaunchKernelGGL(csr_offsets_kernel, dim3(grid_for(atom_count + 1, 256)), dim3(256), 0, as_stream(stream), centers,
+                     edge_count, atom_count, row_offsets);
+  return check_launch("csr_offsets_kernel");
 }
 
 int ye3t_hip_density_accumulate_adjoint(int dtype, const void* adj, const int64_t* centers, int64_t E, int64_t C,
@@ -700,18 +849,16 @@ int ye3t_hip_density_accumulate_adjoint(int dtype, const void* adj, const int64_
                    reinterpret_cast<uintptr_t>(out) % 16 == 0;
   const hipStream_t s = as_stream(stream);
   const int64_t CV = vec ? int64_t(size_t(C) * elem / 16) : C;
-  YE3T_REQUIRE(CV < (int64_t(1) << 30), "channel_count too large");
-  const int64_t epb = CV >= 256 ? 1 : 256 / CV;
-  const unsigned grid = grid_for((E + epb - 1) / epb, 1);
+  const unsigned grid = grid_for(E * CV, 256 * kGatherSteps);
   if (vec) {
     hipLaunchKernelGGL(density_adjoint_kernel<f32x4>, dim3(grid), dim3(256), 0, s, (const f32x4*)adj, centers, E,
-                       int(CV), N, (f32x4*)out);
+                       CV, N, (f32x4*)out);
   } else if (dtype == YE3T_F64) {
     hipLaunchKernelGGL(density_adjoint_kernel<double>, dim3(grid), dim3(256), 0, s, (const double*)adj, centers, E,
-                       int(CV), N, (double*)out);
+                       CV, N, (double*)out);
   } else {
     hipLaunchKernelGGL(density_adjoint_kernel<float>, dim3(grid), dim3(256), 0, s, (const float*)adj, centers, E,
-                       int(CV), N, (float*)out);
+                       CV, N, (float*)out);
   }
   return check_launch("density_adjoint_kernel");
 }

@@ -260,9 +260,14 @@ def _csr_passes(row_offsets, neighbors, atom_count, edge_count, species, species
                             and species_count is not None))
     if not shaped:
         return False
-    found = native.check_indices(row_offsets, atom_count, neighbors, atom_count, species,
-                                 0 if species is None else int(species_count))
-    return found is not None and found[0] == 0 and found[1] == edge_count and not any(found[2:5])
+    checks = [(row_offsets, native.INT64_MIN, native.INT64_MAX, True)]
+    if neighbors is not None:
+        checks.append((neighbors, 0, atom_count, False))
+    if species is not None:
+        checks.append((species, 0, int(species_count), False))
+    found = native.check_indices(*checks)
+    return found is not None and found[0][:2] == (0, edge_count) and not found[0][3] and \
+        not any(bad for _, _, bad, _ in found[1:])
 
 
 def validate_density_csr(row_offsets, neighbors, atom_count, edge_count, *, species=None, species_count=None):
@@ -317,19 +322,20 @@ def density_accumulate(edge_values, centers, atom_count, *, backend="auto"):
         raise ValueError("edge_values must be [E, C] and centers [E]")
     atom_count = int(atom_count)
     centers = centers.to(torch.int64)
-    if centers.numel():
-        lo, hi = int(centers.min()), int(centers.max())
-        if lo < 0 or hi >= atom_count:
-            raise RuntimeError("density_accumulate center index out of range")
-    ordered = bool(centers.numel() < 2 or bool((centers[1:] >= centers[:-1]).all()))
+    found = native.check_indices((centers, 0, atom_count, True)) if centers.is_cuda else None
+    if found is not None:
+        bad, ordered = found[0][2], not found[0][3]
+    else:
+        bad = bool(centers.numel()) and (int(centers.min()) < 0 or int(centers.max()) >= atom_count)
+        ordered = bool(centers.numel() < 2 or bool((centers[1:] >= centers[:-1]).all()))
+    if bad:
+        raise RuntimeError("density_accumulate center index out of range")
     values = edge_values.contiguous()
     if not ordered:
         perm = torch.sort(centers, stable=True).indices
         centers = centers[perm]
         values = values[perm].contiguous()
-    counts = torch.bincount(centers, minlength=atom_count)
-    offsets = torch.zeros(atom_count + 1, dtype=torch.int64, device=values.device)
-    offsets[1:] = torch.cumsum(counts, 0)
+    offsets = native.csr_offsets(centers.to(values.device).contiguous(), atom_count)
     return native.density_accumulate_csr(values, offsets, atom_count)
 
 
@@ -347,10 +353,10 @@ def density_accumulate_adjoint(atomic_adjoint, centers, *, backend="auto"):
     centers = torch.as_tensor(centers, dtype=torch.int64, device=atomic_adjoint.device)
     if atomic_adjoint.ndim != 2 or centers.ndim != 1:
         raise ValueError("atomic_adjoint must be [N, C] and centers [E]")
-    if centers.numel():
-        lo, hi = int(centers.min()), int(centers.max())
-        if lo < 0 or hi >= int(atomic_adjoint.shape[0]):
-            raise RuntimeError("density_accumulate_adjoint center index out of range")
+    rows = int(atomic_adjoint.shape[0])
+    found = native.check_indices((centers, 0, rows, False))
+    if found[0][2] if found is not None else centers.numel() and (int(centers.min()) < 0 or int(centers.max()) >= rows):
+        raise RuntimeError("density_accumulate_adjoint center index out of range")
     return native.density_accumulate_adjoint(atomic_adjoint.contiguous(), centers.contiguous())
 
 

@@ -73,6 +73,11 @@ class CellGrid(ctypes.Structure):
     _fields_ = [("origin", ctypes.c_double * 3), ("cell_edge", ctypes.c_double), ("dims", _i64 * 3)]
 
 
+class IndexCheck(ctypes.Structure):
+    _fields_ = [("data", _vp), ("count", _i64), ("first", _i64), ("limit", _i64), ("width", ctypes.c_int),
+                ("ordered", ctypes.c_int)]
+
+
 class Caps(ctypes.Structure):
     _fields_ = [("arch", ctypes.c_char * 64), ("device", ctypes.c_int), ("cu_count", ctypes.c_int),
                 ("wavefront_size", ctypes.c_int), ("lds_bytes_per_block", ctypes.c_int),
@@ -106,7 +111,8 @@ def lib():
     L.ye3t_hip_scheduled_radial_angular_channels.argtypes = [ctypes.c_int, _i64, _i64, _i64, _i64] + [_vp] * 13
     L.ye3t_hip_density_accumulate_csr.argtypes = [ctypes.c_int, _vp, _vp, _i64, _i64, _vp, _vp]
     L.ye3t_hip_density_accumulate_adjoint.argtypes = [ctypes.c_int, _vp, _vp, _i64, _i64, _i64, _vp, _vp]
-    L.ye3t_hip_check_indices.argtypes = [_vp, _i64, _vp, _i64, _i64, _vp, _i64, ctypes.POINTER(_i64), _vp]
+    L.ye3t_hip_check_indices.argtypes = [ctypes.POINTER(IndexCheck), ctypes.c_int, ctypes.POINTER(_i64), _vp]
+    L.ye3t_hip_csr_offsets.argtypes = [_vp, _i64, _i64, _vp, _vp]
     L.ye3t_hip_ace_density_forward.argtypes = [ctypes.POINTER(DensityArgs), _vp, _vp]
     L.ye3t_hip_ace_density_edge_gradient.argtypes = [ctypes.POINTER(DensityArgs), ctypes.c_int, _vp, _vp, _vp]
     L.ye3t_hip_symmetric_power_monomial.argtypes = [ctypes.c_int, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _i64, _i64,
@@ -226,6 +232,7 @@ EXPORTED_SYMBOLS = (
     "ye3t_hip_symmetric_power_shared_sparse_monomial_adjoint",
     "ye3t_hip_symmetric_power_shared_sparse_monomial_double_backward", "ye3t_hip_code_object_kernel_info",
     "ye3t_hip_part_private_limit", "ye3t_hip_check_indices",
+    "ye3t_hip_csr_offsets",
 )
 
 
@@ -309,7 +316,7 @@ def scheduled_radial_angular_channels(radial_values, radial_derivatives, angular
                                       channel_angular_indices, channel_types, channel_scales):
     """``ye3t_hip_scheduled_radial_angular_channels`` with the reference's
     argument checks and messages (``execution_plan_torch.cpp:1241-1305``);
-    the index ranges are checked by one device reduction each.  Returns
+    the index ranges are checked by one device pass (:func:`check_indices`).  Returns
     ``(edge_values [E, K], edge_derivatives [E, K, 3])``."""
     import torch
 
@@ -339,7 +346,9 @@ def scheduled_radial_angular_channels(radial_values, radial_derivatives, angular
         raise ValueError("edge_types must have length edge_count")
     if not (channel_radial_indices.numel() == channel_angular_indices.numel() == channel_types.numel() == K):
         raise ValueError("channel schedule arrays must have length channel_count")
-    if K > 0:
+    found = check_indices((channel_radial_indices, 0, NR, False), (channel_angular_indices, 0, NA, False),
+                          (channel_types, -1, INT64_MAX, False)) if K > 0 and channel_types.is_cuda else None
+    if K > 0 and (found is None or any(bad for _, _, bad, _ in found)):
         if int(channel_radial_indices.min()) < 0 or int(channel_radial_indices.max()) >= NR:
             raise ValueError("channel radial indices must lie in the radial table")
         if int(channel_angular_indices.min()) < 0 or int(channel_angular_indices.max()) >= NA:
@@ -376,27 +385,42 @@ def real_sph_table(vectors, l_max, epsilon=1e-12, with_gradient=True):
     return values, grads
 
 
-def check_indices(row_offsets, atom_count, indices, limit, species=None, species_count=0):
-    """One device pass over index inputs (``ye3t_hip_check_indices``): the list
-    ``[first offset, last offset, offsets fall, index out of range, species out
-    of range, indices fall]``, or ``None`` where the device cannot answer (a
-    tensor that is not contiguous or not on the current device, a stream under
-    capture).  Waits for the current stream."""
+INT64_MIN, INT64_MAX = -2 ** 63, 2 ** 63 - 1
+
+
+def check_indices(*checks):
+    """One device pass over index vectors (``ye3t_hip_check_indices``).  Each
+    check is ``(tensor, first, limit, ordered)`` of an int32 or int64 tensor;
+    returns one ``(first value, last value, out of range, falls)`` for each, or
+    ``None`` where the device cannot answer (a tensor that is not contiguous or
+    not on the current device, a stream under capture).  Waits for the current
+    stream."""
     import torch
 
     device = torch.cuda.current_device()
-    for t in (row_offsets, indices, species):
-        if t is not None and not (t.is_cuda and t.device.index == device and t.is_contiguous()):
+    asked = (IndexCheck * len(checks))()
+    for c, (t, first, limit, ordered) in zip(asked, checks):
+        if not (t.is_cuda and t.device.index == device and t.is_contiguous()):
             return None
-    result = (_i64 * 6)()
-    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
-    rc = lib().ye3t_hip_check_indices(ptr(row_offsets), atom_count, ptr(indices),
-                                      0 if indices is None else indices.shape[0], limit, ptr(species),
-                                      species_count, result, _stream())
+        c.data, c.count, c.first, c.limit = t.data_ptr(), t.numel(), first, limit
+        c.width, c.ordered = t.element_size(), int(ordered)
+    result = (_i64 * (4 * len(checks)))()
+    rc = lib().ye3t_hip_check_indices(asked, len(checks), result, _stream())
     if rc == EUNSUPPORTED:
         return None
     _check(rc, "ye3t_hip_check_indices")
-    return list(result)
+    return [(result[4 * k], result[4 * k + 1], bool(result[4 * k + 2]), bool(result[4 * k + 3]))
+            for k in range(len(checks))]
+
+
+def csr_offsets(centers, atom_count):
+    """Row offsets ``[atom_count + 1]`` of centres that do not fall and lie in ``[0, atom_count)``."""
+    import torch
+
+    out = torch.empty(atom_count + 1, dtype=torch.int64, device=centers.device)
+    _check(lib().ye3t_hip_csr_offsets(_dev(centers, "centers"), int(centers.shape[0]), int(atom_count),
+                                      _dev(out, "row_offsets"), _stream()), "ye3t_hip_csr_offsets")
+    return out
 
 
 def density_accumulate_csr(edge_values, row_offsets, atom_count):
