@@ -6,9 +6,12 @@
 // (with its second order).  These are the reference's stand-alone ops;
 // the ACE product plan evaluates its symmetric blocks inside its own kernels.
 //
-// Forward: one thread per (row, output).  Adjoints: one thread per row, which
-// owns its row of the input gradient (no atomics, fixed order).  The tables are
-// validated by the caller (ye3t_amd.runtime checks them on the host).
+// Forward and adjoint run on tiles of 64 rows (monomial_tile_*_kernel: lane =
+// row); rows too wide for a tile, and the second order, on one thread per
+// (row, output) or per row.  No atomics, fixed order.  The tables are validated
+// by the caller (ye3t_amd.runtime checks them on the host).
+#include <type_traits>
+
 #include "common.h"
 
 namespace ye3t {
@@ -276,6 +279,281 @@ __global__ __launch_bounds__(256) void sparse_monomial_adjoint_kernel(
   }
 }
 
+// ---- tiles of 64 rows -------------------------------------------------------
+//
+// Lane = row, so that the table, the same for every row, is wave-uniform: no
+// lane waits for another's term.  The rows' components are in LDS (component-major), and so is
+// the table where it fits; the waves of a workgroup share the outputs
+// (forward) or the coefficients (adjoint, each wave with its own gradient rows
+// in LDS, summed in wave order).  Bound by the latency of those short dependent
+// steps, hence as many waves a tile as its gradients leave room for.  70
+// monomials of degree 4 over 5 components, 315 coefficients, 20 000 rows, fp64:
+// forward 68 -> FWD_US us, adjoint 473 -> ADJ_US us (one thread a row, its gradient read
+// and written in memory for every factor).
+
+// One table for the three forms.  Monomial t has factors [begin(t), end(t)),
+// factor q is x[component(q)]^exponent(q); coefficient k combines monomial
+// term(k).
+struct MonomialTable {
+  const int64_t* counts;  // dense: exponents [M, D]; NULL: sparse supports
+  const int64_t* toff;
+  const int64_t* comp;
+  const int64_t* ex;
+  const int64_t* terms;    // NULL: coefficient k is monomial k, which starts from its value
+  const int64_t* outputs;  // output of coefficient k; NULL: by the output offsets
+  int64_t D, M, S, C, O;
+};
+
+constexpr int kTileRows = 64;
+constexpr size_t kTileLds = 64 * 1024;    // rows and gradients of a tile
+constexpr size_t kTableLds = 32 * 1024;   // table held beside them
+
+__device__ inline int64_t uniform64(int64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(int(uint32_t(uint64_t(v))));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(int(uint32_t(uint64_t(v) >> 32)));
+  return int64_t((uint64_t(hi) << 32) | lo);
+}
+
+template <typename Real>
+__device__ inline Real uniform_value(Real v) {
+  if constexpr (sizeof(Real) == 4) {
+    return __builtin_bit_cast(Real, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+  } else if constexpr (sizeof(Real) == 8) {
+    return __builtin_bit_cast(Real, uniform64(__builtin_bit_cast(int64_t, v)));
+  } else {
+    return {uniform_value(v.re), uniform_value(v.im)};
+  }
+}
+
+// The table's arrays in LDS (copied by the whole workgroup) or in memory.
+struct HeldTable {
+  const int64_t *exps, *comp, *toff, *terms, *outputs, *offsets;
+  const void* values;
+};
+
+inline size_t held_bytes(const MonomialTable& t, size_t elem) {
+  const int64_t words = (t.counts ? t.M * t.D : t.M + 1 + 2 * t.S) + (t.terms ? t.C : 0) + (t.outputs ? t.C : t.O + 1);
+  return size_t(words) * 8 + size_t(t.C) * elem;
+}
+
+template <bool HELD, typename Real>
+__device__ inline HeldTable hold_table(const MonomialTable& t, const int64_t* offsets, const Real* values,
+                                       unsigned char* lds) {
+  if (!HELD) return {t.counts ? t.counts : t.ex, t.comp, t.toff, t.terms, t.outputs, offsets, values};
+  auto copy = [&](const auto* from, int64_t n) {
+    using T = std::remove_cv_t<std::remove_reference_t<decltype(*from)>>;
+    T* to = reinterpret_cast<T*>(lds);
+    lds += size_t(n) * sizeof(T);
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) to[i] = from[i];
+    return static_cast<const T*>(to);
+  };
+  HeldTable h = {};
+  h.exps = t.counts ? copy(t.counts, t.M * t.D) : copy(t.ex, t.S);
+  if (!t.counts) {
+    h.comp = copy(t.comp, t.S);
+    h.toff = copy(t.toff, t.M + 1);
+  }
+  if (t.terms) h.terms = copy(t.terms, t.C);
+  if (t.outputs) h.outputs = copy(t.outputs, t.C);
+  if (offsets) h.offsets = copy(offsets, t.O + 1);
+  h.values = copy(values, t.C);  // last: an odd number of 4-byte values would misalign what follows
+  return h;
+}
+
+template <bool DENSE>
+__device__ inline void factor_range(const MonomialTable& t, const HeldTable& h, int64_t m, int64_t& q0, int64_t& q1) {
+  q0 = DENSE ? m * t.D : uniform64(h.toff[m]);
+  q1 = DENSE ? (m + 1) * t.D : uniform64(h.toff[m + 1]);
+}
+
+// rows of x into xs[component][row]; rows past the batch hold ones
+template <typename Real>
+__device__ inline void load_rows(const Real* __restrict__ x, int64_t b0, int64_t batch, int64_t D, Real* xs) {
+  for (int64_t i = threadIdx.x; i < kTileRows * D; i += blockDim.x) {
+    const int64_t r = i / D, c = i - r * D;
+    xs[c * kTileRows + r] = b0 + r < batch ? x[(b0 + r) * D + c] : Real(1);
+  }
+}
+
+template <bool DENSE, bool HELD, typename Real>
+__global__ __launch_bounds__(512) void monomial_tile_kernel(const Real* __restrict__ x, int64_t batch, MonomialTable t,
+                                                            const int64_t* __restrict__ offsets,
+                                                            const Real* __restrict__ values, Real* __restrict__ out) {
+  extern __shared__ __align__(16) unsigned char tile_smem[];
+  Real* const xs = reinterpret_cast<Real*>(tile_smem);
+  const int64_t b0 = int64_t(blockIdx.x) * kTileRows;
+  const int lane = threadIdx.x & 63;
+  const int waves = int(blockDim.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const HeldTable h =
+      hold_table<HELD>(t, offsets, values, tile_smem + size_t(t.D) * kTileRows * sizeof(Real));
+  const Real* const hv = static_cast<const Real*>(h.values);
+  load_rows(x, b0, batch, t.D, xs);
+  __syncthreads();
+  for (int64_t o = wave; o < t.O; o += waves) {
+    const int64_t k1 = uniform64(h.offsets[o + 1]);
+    Real acc = Real(0);
+    for (int64_t k = uniform64(h.offsets[o]); k < k1; ++k) {
+      const Real v = uniform_value(hv[k]);
+      const int64_t m = t.terms ? uniform64(h.terms[k]) : k;
+      int64_t q0, q1;
+      factor_range<DENSE>(t, h, m, q0, q1);
+      Real p = t.terms ? Real(1) : v;
+      for (int64_t q = q0; q < q1; ++q) {
+        const int64_t e = uniform64(h.exps[q]);
+        if (e == 0) continue;
+        p *= ipow(xs[(DENSE ? q - q0 : uniform64(h.comp[q])) * kTileRows + lane], e);
+      }
+      if (t.terms) acc += v * p;
+      else acc += p;
+    }
+    if (b0 + lane < batch) out[(b0 + lane) * t.O + o] = acc;
+  }
+}
+
+// Input gradient, with the zero-factor rules of monomial_gradient (dense: a
+// single zero factor of exponent one takes the cofactor) and of
+// sparse_monomial_adjoint_kernel, which are one: a zero degree of one.
+template <bool DENSE, bool HELD, typename Real>
+__global__ __launch_bounds__(512) void monomial_tile_adjoint_kernel(
+    const Real* __restrict__ gout, const Real* __restrict__ x, int64_t batch, MonomialTable t,
+    const int64_t* __restrict__ offsets, const Real* __restrict__ values, Real* __restrict__ gin) {
+  extern __shared__ __align__(16) unsigned char tile_smem[];
+  const int64_t size = t.D * kTileRows;
+  Real* const xs = reinterpret_cast<Real*>(tile_smem);
+  const int64_t b0 = int64_t(blockIdx.x) * kTileRows;
+  const int lane = threadIdx.x & 63;
+  const int waves = int(blockDim.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  Real* const grads = xs + size;
+  Real* const grad = grads + wave * size;
+  const HeldTable h =
+      hold_table<HELD>(t, offsets, values, tile_smem + size_t(size) * size_t(1 + waves) * sizeof(Real));
+  const Real* const hv = static_cast<const Real*>(h.values);
+  load_rows(x, b0, batch, t.D, xs);
+  for (int64_t i = threadIdx.x; i < size * waves; i += blockDim.x) grads[i] = Real(0);
+  __syncthreads();
+  const int64_t b = b0 + lane < batch ? b0 + lane : batch - 1;
+  const int64_t k0 = t.C * wave / waves, k1 = t.C * (wave + 1) / waves;
+  // the output before the wave's first coefficient's, and where it ends
+  int64_t o = -1, end = k0;
+  if (!t.outputs && k0 < k1) {
+    int64_t lo = 0, hi = t.O;
+    while (hi - lo > 1) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (uniform64(h.offsets[mid]) <= k0) lo = mid;
+      else hi = mid;
+    }
+    o = lo - 1;
+  }
+  Real g = Real(0);
+  for (int64_t k = k0; k < k1; ++k) {
+    const int64_t before = o;
+    if (t.outputs) {
+      o = uniform64(h.outputs[k]);
+    } else {
+      while (k >= end) end = uniform64(h.offsets[++o + 1]);
+    }
+    if (o != before) g = gout[b * t.O + o];
+    const Real v = uniform_value(hv[k]);
+    const int64_t m = t.terms ? uniform64(h.terms[k]) : k;
+    int64_t q0, q1;
+    factor_range<DENSE>(t, h, m, q0, q1);
+    const Real w = g * conjv(v);
+    Real mono = Real(1);
+    int64_t zdeg = 0;  // exponents of the zero factors (dense: those past one factor make it two or more)
+    int64_t zc = 0;
+    for (int64_t q = q0; q < q1; ++q) {
+      const int64_t e = uniform64(h.exps[q]);
+      if (e == 0) continue;
+      const int64_t c = DENSE ? q - q0 : uniform64(h.comp[q]);
+      const Real xv = xs[c * kTileRows + lane];
+      if (xv == Real(0)) {
+        zdeg += e;
+        zc = c;
+      } else {
+        mono *= ipow(xv, e);
+      }
+    }
+    if (zdeg == 0) {
+      for (int64_t q = q0; q < q1; ++q) {
+        const int64_t e = uniform64(h.exps[q]);
+        if (e == 0) continue;
+        const int64_t c = DENSE ? q - q0 : uniform64(h.comp[q]);
+        grad[c * kTileRows + lane] += w * conjv(Real(e) * mono / xs[c * kTileRows + lane]);
+      }
+    } else if (zdeg == 1) {
+      grad[zc * kTileRows + lane] += w * conjv(mono);
+    }
+  }
+  __syncthreads();
+  for (int64_t i = threadIdx.x; i < size; i += blockDim.x) {
+    const int64_t r = i / t.D, c = i - r * t.D;
+    if (b0 + r >= batch) break;
+    Real sum = grads[c * kTileRows + r];
+    for (int k = 1; k < waves; ++k) sum += grads[k * size + c * kTileRows + r];
+    gin[(b0 + r) * t.D + c] = sum;
+  }
+}
+
+// Launches a tile kernel; YE3T_EUNSUPPORTED, with nothing launched, where a
+// tile of rows (and one wave's gradients) does not fit in kTileLds.
+template <typename Real>
+int launch_tiles(const Real* gout, const Real* x, int64_t batch, const MonomialTable& t, const int64_t* offsets,
+                 const Real* values, Real* out, hipStream_t s) {
+  const size_t rows = size_t(t.D) * kTileRows * sizeof(Real);
+  const int64_t tiles = (batch + kTileRows - 1) / kTileRows;
+  if (t.D < 1 || t.O < 1 || t.D > 1024 || tiles > INT32_MAX) return YE3T_EUNSUPPORTED;
+  int waves = 8;
+  while (waves > 0 && rows * size_t(1 + (gout ? waves : 0)) > kTileLds) waves /= 2;
+  if (waves == 0) return YE3T_EUNSUPPORTED;
+  if (!gout && t.O < waves) waves = int(t.O);
+  const size_t held = held_bytes(t, sizeof(Real));
+  const bool hold = held <= kTableLds;
+  const size_t lds = rows * size_t(1 + (gout ? waves : 0)) + (hold ? held : 0);
+  const dim3 grid{unsigned(tiles)}, block{unsigned(64 * waves)};
+  auto launch = [&](auto dense, auto keep) {
+    if (gout) {
+      auto* const kernel = &monomial_tile_adjoint_kernel<dense.value, keep.value, Real>;
+      if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess) {
+        (void)hipGetLastError();
+        return int(YE3T_EUNSUPPORTED);
+      }
+      hipLaunchKernelGGL((monomial_tile_adjoint_kernel<dense.value, keep.value, Real>), grid, block, lds, s, gout, x,
+                         batch, t, offsets, values, out);
+      return check_launch("monomial_tile_adjoint_kernel");
+    }
+    auto* const kernel = &monomial_tile_kernel<dense.value, keep.value, Real>;
+    if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess) {
+      (void)hipGetLastError();
+      return int(YE3T_EUNSUPPORTED);
+    }
+    hipLaunchKernelGGL((monomial_tile_kernel<dense.value, keep.value, Real>), grid, block, lds, s, x, batch, t, offsets,
+                       values, out);
+    return check_launch("monomial_tile_kernel");
+  };
+  if (t.counts) return hold ? launch(std::true_type{}, std::true_type{}) : launch(std::true_type{}, std::false_type{});
+  return hold ? launch(std::false_type{}, std::true_type{}) : launch(std::false_type{}, std::false_type{});
+}
+
+int launch_tiles(int dtype, const void* gout, const void* x, int64_t batch, const MonomialTable& t,
+                 const int64_t* offsets, const void* values, void* out, hipStream_t s) {
+  auto as = [&](auto zero) {
+    using Real = decltype(zero);
+    return launch_tiles<Real>(static_cast<const Real*>(gout), static_cast<const Real*>(x), batch, t, offsets,
+                              static_cast<const Real*>(values), static_cast<Real*>(out), s);
+  };
+  switch (dtype) {
+    case YE3T_F64: return as(double{});
+    case YE3T_F32: return as(float{});
+    case YE3T_C128: return as(cplx<double>{});
+    case YE3T_C64: return as(cplx<float>{});
+    default: return YE3T_EUNSUPPORTED;
+  }
+}
+
 // Directional derivative of monomial t along v.
 template <typename Real>
 __device__ inline Real sparse_directional(const Real* __restrict__ row, const Real* __restrict__ v,
@@ -372,6 +650,11 @@ int ye3t_hip_symmetric_power_monomial(int dtype, const void* x, int64_t batch, i
   YE3T_REQUIRE(batch >= 0 && D >= 0 && O >= 0 && T >= 0, "negative size");
   if (batch * O == 0) return YE3T_OK;
   YE3T_REQUIRE(x && offsets && out && (T == 0 || (counts && values && output_indices)), "NULL argument");
+  if ((dtype == YE3T_F64 || dtype == YE3T_F32) && T > 0) {
+    const MonomialTable t = {counts, nullptr, nullptr, nullptr, nullptr, nullptr, D, T, 0, T, O};
+    const int rc = launch_tiles(dtype, nullptr, x, batch, t, offsets, values, out, as_stream(stream));
+    if (rc != YE3T_EUNSUPPORTED) return rc;
+  }
   const unsigned grid = grid_for(batch * O, 256);
   if (dtype == YE3T_F64) {
     hipLaunchKernelGGL(sym_monomial_kernel<double>, dim3(grid), dim3(256), 0, as_stream(stream), (const double*)x,
@@ -394,6 +677,11 @@ int ye3t_hip_symmetric_power_monomial_adjoint(int dtype, const void* output_adjo
   if (batch * D == 0) return YE3T_OK;
   YE3T_REQUIRE(x && input_adjoint && (T == 0 || (output_adjoint && counts && values && output_indices)),
                "NULL argument");
+  if ((dtype == YE3T_F64 || dtype == YE3T_F32) && T > 0) {
+    const MonomialTable t = {counts, nullptr, nullptr, nullptr, nullptr, output_indices, D, T, 0, T, O};
+    const int rc = launch_tiles(dtype, output_adjoint, x, batch, t, nullptr, values, input_adjoint, as_stream(stream));
+    if (rc != YE3T_EUNSUPPORTED) return rc;
+  }
   const unsigned grid = grid_for(batch, 256);
   if (dtype == YE3T_F64) {
     hipLaunchKernelGGL(sym_monomial_adjoint_kernel<double>, dim3(grid), dim3(256), 0, as_stream(stream),
@@ -418,6 +706,11 @@ int ye3t_hip_symmetric_power_shared_monomial(int dtype, const void* x, int64_t b
   if (batch * O == 0) return YE3T_OK;
   YE3T_REQUIRE(x && output_offsets && out && (C == 0 || (counts && coefficient_terms && coefficient_values)),
                "NULL argument");
+  if ((dtype == YE3T_F64 || dtype == YE3T_F32) && C > 0) {
+    const MonomialTable t = {counts, nullptr, nullptr, nullptr, coefficient_terms, nullptr, D, M, 0, C, O};
+    const int rc = launch_tiles(dtype, nullptr, x, batch, t, output_offsets, coefficient_values, out, as_stream(stream));
+    if (rc != YE3T_EUNSUPPORTED) return rc;
+  }
   const unsigned grid = grid_for(batch * O, 256);
   if (dtype == YE3T_F64) {
     hipLaunchKernelGGL(shared_monomial_kernel<double>, dim3(grid), dim3(256), 0, as_stream(stream), (const double*)x,
@@ -445,6 +738,12 @@ int ye3t_hip_symmetric_power_shared_monomial_adjoint(int dtype, const void* outp
   YE3T_REQUIRE(x && input_adjoint && output_offsets &&
                    (C == 0 || (output_adjoint && counts && coefficient_terms && coefficient_values)),
                "NULL argument");
+  if ((dtype == YE3T_F64 || dtype == YE3T_F32) && C > 0) {
+    const MonomialTable t = {counts, nullptr, nullptr, nullptr, coefficient_terms, nullptr, D, M, 0, C, O};
+    const int rc = launch_tiles(dtype, output_adjoint, x, batch, t, output_offsets, coefficient_values, input_adjoint,
+                                as_stream(stream));
+    if (rc != YE3T_EUNSUPPORTED) return rc;
+  }
   const unsigned grid = grid_for(batch, 256);
   if (dtype == YE3T_F64) {
     hipLaunchKernelGGL(shared_monomial_adjoint_kernel<double>, dim3(grid), dim3(256), 0, as_stream(stream),
@@ -492,6 +791,11 @@ int ye3t_hip_symmetric_power_shared_sparse_monomial(int dtype, const void* x, in
   YE3T_REQUIRE(x && output_offsets && out && term_offsets &&
                    (C == 0 || (coefficient_terms && coefficient_values)) && (S == 0 || (term_components && term_exponents)),
                "NULL argument");
+  if (C > 0) {
+    const MonomialTable t = {nullptr, term_offsets, term_components, term_exponents, coefficient_terms, nullptr, D, M, S, C, O};
+    const int rc = launch_tiles(dtype, nullptr, x, batch, t, output_offsets, coefficient_values, out, as_stream(stream));
+    if (rc != YE3T_EUNSUPPORTED) return rc;
+  }
   SPARSE_DISPATCH(sparse_monomial_kernel, grid_for(batch * O, 256), (const Real*)x, batch, D, term_offsets,
                   term_components, term_exponents, output_offsets, coefficient_terms, (const Real*)coefficient_values,
                   O, (Real*)out);
@@ -511,6 +815,12 @@ int ye3t_hip_symmetric_power_shared_sparse_monomial_adjoint(
                    (C == 0 || (output_adjoint && coefficient_terms && coefficient_values)) &&
                    (S == 0 || (term_components && term_exponents)),
                "NULL argument");
+  if (C > 0) {
+    const MonomialTable t = {nullptr, term_offsets, term_components, term_exponents, coefficient_terms, nullptr, D, M, S, C, O};
+    const int rc = launch_tiles(dtype, output_adjoint, x, batch, t, output_offsets, coefficient_values, input_adjoint,
+                                as_stream(stream));
+    if (rc != YE3T_EUNSUPPORTED) return rc;
+  }
   SPARSE_DISPATCH(sparse_monomial_adjoint_kernel, grid_for(batch, 256), (const Real*)output_adjoint, (const Real*)x,
                   batch, D, term_offsets, term_components, term_exponents, output_offsets, coefficient_terms,
                   (const Real*)coefficient_values, O, (Real*)input_adjoint);

@@ -439,45 +439,43 @@ def neighbor_list(positions, cutoff, *, backend="auto"):
 def _monomial_functions():
     import torch
 
+    # a call's tables are checked and copied once: the gradient uses the forward's
     class _Grouped(torch.autograd.Function):
         @staticmethod
         def forward(ctx, x, counts, offsets, indices, values):
             ctx.save_for_backward(x)
-            ctx.table = (counts, offsets, indices, values)
-            return native.symmetric_power_monomial(x, counts, offsets, values, output_indices=indices)
+            ctx.table = native.GroupedTable(x, counts, offsets, values, indices)
+            return ctx.table.forward(x)
 
         @staticmethod
         def backward(ctx, g):
             (x,) = ctx.saved_tensors
-            counts, offsets, indices, values = ctx.table
-            return native.symmetric_power_monomial_adjoint(g.contiguous(), x, counts, indices, values,
-                                                           offsets), None, None, None, None
+            return ctx.table.adjoint(g.contiguous(), x), None, None, None, None
 
     class _Shared(torch.autograd.Function):
         @staticmethod
         def forward(ctx, x, counts, offsets, terms, outputs, values):
             ctx.save_for_backward(x)
-            ctx.table = (counts, offsets, terms, outputs, values)
-            return native.symmetric_power_shared_monomial(x, counts, offsets, terms, outputs, values)
+            ctx.table = native.SharedTable(x, counts, offsets, terms, outputs, values)
+            return ctx.table.forward(x)
 
         @staticmethod
         def backward(ctx, g):
             (x,) = ctx.saved_tensors
-            return (native.symmetric_power_shared_monomial_adjoint(g.contiguous(), x, *ctx.table),
-                    None, None, None, None, None)
+            return ctx.table.adjoint(g.contiguous(), x), None, None, None, None, None
 
     class _Sparse(torch.autograd.Function):
         @staticmethod
         def forward(ctx, x, *tables):
             ctx.save_for_backward(x)
-            ctx.table = tables
-            return native.symmetric_power_shared_sparse_monomial(x, *tables)
+            ctx.table = native.SparseMonomialTable(x.shape[1], *tables, device=x.device, dtype=x.dtype)
+            ctx.arguments = len(tables)
+            return ctx.table.forward(x)
 
         @staticmethod
         def backward(ctx, g):
             (x,) = ctx.saved_tensors
-            return (native.symmetric_power_shared_sparse_monomial_adjoint(g.contiguous(), x, *ctx.table),) + \
-                (None,) * len(ctx.table)
+            return (ctx.table.adjoint(g.contiguous(), x),) + (None,) * ctx.arguments
 
     return _Grouped, _Shared, _Sparse
 

@@ -636,85 +636,126 @@ def _dev_i64(a, device):
     return torch.as_tensor(a, dtype=torch.int64, device=device).contiguous()
 
 
+def _upload(device, dtype, values, *ints):
+    """int64 arrays and the values in ``dtype`` on ``device``: one copy, returned
+    as views of it, the values last (an upload each is as many waits)."""
+    import torch
+
+    values = torch.as_tensor(_host_real(values)).reshape(-1).to(dtype).numpy()
+    parts = [np.ascontiguousarray(a, dtype=np.int64).reshape(-1) for a in ints] + [values]
+    ends = np.cumsum([(a.nbytes + 15) // 16 * 16 for a in parts])
+    host = np.empty(int(ends[-1]), dtype=np.uint8)
+    for a, end in zip(parts, ends):
+        start = int(end) - (a.nbytes + 15) // 16 * 16
+        host[start:start + a.nbytes] = a.view(np.uint8)
+    there = torch.from_numpy(host).to(device)
+    out = []
+    for a, end in zip(parts, ends):
+        start = int(end) - (a.nbytes + 15) // 16 * 16
+        out.append(there[start:start + a.nbytes].view(torch.int64 if len(out) < len(ints) else dtype))
+    return out
+
+
+def _ptr(t):
+    return t.data_ptr() if t.numel() else None
+
+
+class GroupedTable:
+    """A grouped monomial table, validated and on one device in one dtype, for
+    one call and its gradient."""
+
+    def __init__(self, x, counts, offsets, values, indices=None):
+        if indices is None:
+            offs = _host_i64(offsets).reshape(-1)
+            indices = np.repeat(np.arange(offs.size - 1), np.diff(offs))
+        counts, offs, idx = check_monomial_table(int(x.shape[1]), counts, offsets, indices, values)
+        self.T, self.O = int(counts.shape[0]), int(offs.size - 1)
+        self.arrays = _upload(x.device, x.dtype, values, counts, offs, idx)
+
+    def forward(self, x):
+        import torch
+
+        B, D = (int(s) for s in x.shape)
+        out = torch.empty((B, self.O), dtype=x.dtype, device=x.device)
+        counts, offs, idx, values = (_ptr(t) for t in self.arrays)
+        _check(lib().ye3t_hip_symmetric_power_monomial(_dtype_code(x), _dev(x, "input"), B, D, counts, offs, idx, values,
+                                                       self.T, self.O, _dev(out, "out"), _stream()),
+               "ye3t_hip_symmetric_power_monomial")
+        return out
+
+    def adjoint(self, output_adjoint, x):
+        import torch
+
+        B, D = (int(s) for s in x.shape)
+        g = output_adjoint.to(x.dtype).contiguous()
+        if tuple(g.shape) != (B, self.O):
+            raise ValueError(f"output_adjoint must be [{B}, {self.O}]")
+        out = torch.empty_like(x)
+        counts, _, idx, values = (_ptr(t) for t in self.arrays)
+        _check(lib().ye3t_hip_symmetric_power_monomial_adjoint(_dtype_code(x), _dev(g, "output_adjoint"),
+                                                               _dev(x, "input"), B, D, counts, idx, values, self.T,
+                                                               self.O, _dev(out, "input_adjoint"), _stream()),
+               "ye3t_hip_symmetric_power_monomial_adjoint")
+        return out
+
+
+class SharedTable:
+    """A shared monomial table, as :class:`GroupedTable`."""
+
+    def __init__(self, x, counts, offsets, terms, outputs, values):
+        counts, offs, terms, _ = check_shared_table(int(x.shape[1]), counts, offsets, terms, outputs, values)
+        self.M, self.C, self.O = int(counts.shape[0]), int(terms.size), int(offs.size - 1)
+        self.arrays = _upload(x.device, x.dtype, values, counts, offs, terms)
+
+    def _args(self):
+        counts, offs, terms, values = (_ptr(t) for t in self.arrays)
+        return counts, self.M, offs, terms, values, self.C, self.O
+
+    def forward(self, x):
+        import torch
+
+        B, D = (int(s) for s in x.shape)
+        out = torch.empty((B, self.O), dtype=x.dtype, device=x.device)
+        _check(lib().ye3t_hip_symmetric_power_shared_monomial(_dtype_code(x), _dev(x, "input"), B, D, *self._args(),
+                                                              _dev(out, "out"), _stream()),
+               "ye3t_hip_symmetric_power_shared_monomial")
+        return out
+
+    def adjoint(self, output_adjoint, x):
+        import torch
+
+        B, D = (int(s) for s in x.shape)
+        g = output_adjoint.to(x.dtype).contiguous()
+        if tuple(g.shape) != (B, self.O):
+            raise ValueError(f"output_adjoint must be [{B}, {self.O}]")
+        out = torch.empty_like(x)
+        _check(lib().ye3t_hip_symmetric_power_shared_monomial_adjoint(
+            _dtype_code(x), _dev(g, "output_adjoint"), _dev(x, "input"), B, D, *self._args(),
+            _dev(out, "input_adjoint"), _stream()), "ye3t_hip_symmetric_power_shared_monomial_adjoint")
+        return out
+
+
 def symmetric_power_monomial(x, monomial_counts, output_offsets, monomial_values, output_indices=None):
     """Grouped monomial table on the device (``output_indices`` defaults to the
     offsets' own term-to-output map)."""
-    import torch
-
-    B, D = (int(s) for s in x.shape)
-    if output_indices is None:
-        offs = _host_i64(output_offsets).reshape(-1)
-        output_indices = np.repeat(np.arange(offs.size - 1), np.diff(offs))
-    counts, offs, idx = check_monomial_table(D, monomial_counts, output_offsets, output_indices, monomial_values)
-    T, O = int(counts.shape[0]), int(offs.size - 1)
-    out = torch.empty((B, O), dtype=x.dtype, device=x.device)
-    dv = torch.as_tensor(_host_real(monomial_values), device=x.device).to(x.dtype).contiguous()
-    dc, do, di = _dev_i64(counts, x.device), _dev_i64(offs, x.device), _dev_i64(idx, x.device)
-    _check(lib().ye3t_hip_symmetric_power_monomial(_dtype_code(x), _dev(x, "input"), B, D, _dev(dc, "counts"),
-                                                   _dev(do, "offsets"), _dev(di, "indices"), _dev(dv, "values"), T, O,
-                                                   _dev(out, "out"), _stream()), "ye3t_hip_symmetric_power_monomial")
-    return out
+    return GroupedTable(x, monomial_counts, output_offsets, monomial_values, output_indices).forward(x)
 
 
 def symmetric_power_monomial_adjoint(output_adjoint, x, monomial_counts, output_indices, monomial_values,
                                      output_offsets):
-    import torch
-
-    B, D = (int(s) for s in x.shape)
-    counts, offs, idx = check_monomial_table(D, monomial_counts, output_offsets, output_indices, monomial_values)
-    T, O = int(counts.shape[0]), int(offs.size - 1)
-    g = output_adjoint.to(x.dtype).contiguous()
-    if tuple(g.shape) != (B, O):
-        raise ValueError(f"output_adjoint must be [{B}, {O}]")
-    out = torch.empty_like(x)
-    dv = torch.as_tensor(_host_real(monomial_values), device=x.device).to(x.dtype).contiguous()
-    dc, di = _dev_i64(counts, x.device), _dev_i64(idx, x.device)
-    _check(lib().ye3t_hip_symmetric_power_monomial_adjoint(_dtype_code(x), _dev(g, "output_adjoint"),
-                                                           _dev(x, "input"), B, D, _dev(dc, "counts"),
-                                                           _dev(di, "indices"), _dev(dv, "values"), T, O,
-                                                           _dev(out, "input_adjoint"), _stream()),
-           "ye3t_hip_symmetric_power_monomial_adjoint")
-    return out
+    return GroupedTable(x, monomial_counts, output_offsets, monomial_values, output_indices).adjoint(output_adjoint, x)
 
 
 def symmetric_power_shared_monomial(x, monomial_counts, output_offsets, coefficient_terms, coefficient_outputs,
                                     coefficient_values):
-    import torch
-
-    B, D = (int(s) for s in x.shape)
-    counts, offs, terms, _ = check_shared_table(D, monomial_counts, output_offsets, coefficient_terms,
-                                                coefficient_outputs, coefficient_values)
-    M, C, O = int(counts.shape[0]), int(terms.size), int(offs.size - 1)
-    out = torch.empty((B, O), dtype=x.dtype, device=x.device)
-    dv = torch.as_tensor(_host_real(coefficient_values), device=x.device).to(x.dtype).contiguous()
-    dc, do, dt = _dev_i64(counts, x.device), _dev_i64(offs, x.device), _dev_i64(terms, x.device)
-    _check(lib().ye3t_hip_symmetric_power_shared_monomial(_dtype_code(x), _dev(x, "input"), B, D,
-                                                          _dev(dc, "counts") if M else None, M, _dev(do, "offsets"),
-                                                          _dev(dt, "terms") if C else None,
-                                                          _dev(dv, "values") if C else None, C, O, _dev(out, "out"),
-                                                          _stream()), "ye3t_hip_symmetric_power_shared_monomial")
-    return out
+    return SharedTable(x, monomial_counts, output_offsets, coefficient_terms, coefficient_outputs,
+                       coefficient_values).forward(x)
 
 
 def symmetric_power_shared_monomial_adjoint(output_adjoint, x, monomial_counts, output_offsets, coefficient_terms,
                                             coefficient_outputs, coefficient_values):
-    import torch
-
-    B, D = (int(s) for s in x.shape)
-    counts, offs, terms, _ = check_shared_table(D, monomial_counts, output_offsets, coefficient_terms,
-                                                coefficient_outputs, coefficient_values)
-    M, C, O = int(counts.shape[0]), int(terms.size), int(offs.size - 1)
-    g = output_adjoint.to(x.dtype).contiguous()
-    if tuple(g.shape) != (B, O):
-        raise ValueError(f"output_adjoint must be [{B}, {O}]")
-    out = torch.empty_like(x)
-    dv = torch.as_tensor(_host_real(coefficient_values), device=x.device).to(x.dtype).contiguous()
-    dc, do, dt = _dev_i64(counts, x.device), _dev_i64(offs, x.device), _dev_i64(terms, x.device)
-    _check(lib().ye3t_hip_symmetric_power_shared_monomial_adjoint(
-        _dtype_code(x), _dev(g, "output_adjoint"), _dev(x, "input"), B, D, _dev(dc, "counts") if M else None, M,
-        _dev(do, "offsets"), _dev(dt, "terms") if C else None, _dev(dv, "values") if C else None, C, O,
-        _dev(out, "input_adjoint"), _stream()), "ye3t_hip_symmetric_power_shared_monomial_adjoint")
-    return out
+    return SharedTable(x, monomial_counts, output_offsets, coefficient_terms, coefficient_outputs,
+                       coefficient_values).adjoint(output_adjoint, x)
 
 
 def check_sparse_table(D, term_offsets, term_components, term_exponents, output_offsets, coefficient_terms,
@@ -756,16 +797,10 @@ def check_sparse_table(D, term_offsets, term_components, term_exponents, output_
 def _sparse_call(fn_name, x, tables, *tensors_before, outputs):
     toff, comp, ex, offs, terms, values = tables
     M, S, C, O = int(toff.size - 1), int(comp.size), int(terms.size), int(offs.size - 1)
-    import torch
-
-    dv = torch.as_tensor(_host_real(values), device=x.device).to(x.dtype).contiguous()
-    dt, dc, de = _dev_i64(toff, x.device), _dev_i64(comp, x.device), _dev_i64(ex, x.device)
-    do, dk = _dev_i64(offs, x.device), _dev_i64(terms, x.device)
+    dt, dc, de, do, dk, dv = _upload(x.device, x.dtype, values, toff, comp, ex, offs, terms)
     B, D = (int(s) for s in x.shape)
     args = [_any_dtype_code(x.dtype), *[_dev(t, "tensor") for t in tensors_before], _dev(x, "input"), B, D,
-            _dev(dt, "term_offsets"), _dev(dc, "term_components") if S else None,
-            _dev(de, "term_exponents") if S else None, M, S, _dev(do, "output_offsets"),
-            _dev(dk, "coefficient_terms") if C else None, _dev(dv, "coefficient_values") if C else None, C, O,
+            _ptr(dt), _ptr(dc), _ptr(de), M, S, _ptr(do), _ptr(dk), _ptr(dv), C, O,
             *[_dev(t, "output") if t.numel() else None for t in outputs], _stream()]
     _check(getattr(lib(), fn_name)(*args), fn_name)
 
@@ -786,13 +821,8 @@ class SparseMonomialTable:
         self.M, self.S, self.C, self.O = int(toff.size - 1), int(comp.size), int(terms.size), int(offs.size - 1)
         self.dtype = dtype
         self.code = _any_dtype_code(dtype)
-        self.term_offsets = _dev_i64(toff, device)
-        self.term_components = _dev_i64(comp, device)
-        self.term_exponents = _dev_i64(ex, device)
-        self.output_offsets = _dev_i64(offs, device)
-        self.coefficient_terms = _dev_i64(terms, device)
-        self.coefficient_values = torch.as_tensor(_host_real(coefficient_values)).to(device=device,
-                                                                                     dtype=dtype).contiguous()
+        (self.term_offsets, self.term_components, self.term_exponents, self.output_offsets, self.coefficient_terms,
+         self.coefficient_values) = _upload(device, dtype, coefficient_values, toff, comp, ex, offs, terms)
 
     def _args(self):
         return (_dev(self.term_offsets, "term_offsets"),
