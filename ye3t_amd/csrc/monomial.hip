@@ -285,11 +285,12 @@ __global__ __launch_bounds__(256) void sparse_monomial_adjoint_kernel(
 // lane waits for another's term.  The rows' components are in LDS (component-major), and so is
 // the table where it fits; the waves of a workgroup share the outputs
 // (forward) or the coefficients (adjoint, each wave with its own gradient rows
-// in LDS, summed in wave order).  Bound by the latency of those short dependent
+// in LDS, summed in wave order).  Small exponents of few components are packed
+// into one word a monomial.  Bound by the latency of those short dependent
 // steps, hence as many waves a tile as its gradients leave room for.  70
 // monomials of degree 4 over 5 components, 315 coefficients, 20 000 rows, fp64:
-// forward 68 -> FWD_US us, adjoint 473 -> ADJ_US us (one thread a row, its gradient read
-// and written in memory for every factor).
+// forward 68 -> 46 us, adjoint 473 -> 61 us (one thread a row, its gradient read
+// and written in memory for every factor; 65 and 82 us with the exponents unpacked).
 
 // One table for the three forms.  Monomial t has factors [begin(t), end(t)),
 // factor q is x[component(q)]^exponent(q); coefficient k combines monomial
@@ -307,6 +308,7 @@ struct MonomialTable {
 constexpr int kTileRows = 64;
 constexpr size_t kTileLds = 64 * 1024;    // rows and gradients of a tile
 constexpr size_t kTableLds = 32 * 1024;   // table held beside them
+constexpr int64_t kPackedComponents = 16;
 
 __device__ inline int64_t uniform64(int64_t v) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane(int(uint32_t(uint64_t(v))));
@@ -327,19 +329,20 @@ __device__ inline Real uniform_value(Real v) {
 
 // The table's arrays in LDS (copied by the whole workgroup) or in memory.
 struct HeldTable {
+  const uint64_t* packed;  // dense, held, at most kPackedComponents components, exponents below 16: four bits each
   const int64_t *exps, *comp, *toff, *terms, *outputs, *offsets;
   const void* values;
 };
 
 inline size_t held_bytes(const MonomialTable& t, size_t elem) {
-  const int64_t words = (t.counts ? t.M * t.D : t.M + 1 + 2 * t.S) + (t.terms ? t.C : 0) + (t.outputs ? t.C : t.O + 1);
+  const int64_t words = (t.counts ? t.M * t.D + (t.D <= kPackedComponents ? t.M + 1 : 0) : t.M + 1 + 2 * t.S) + (t.terms ? t.C : 0) + (t.outputs ? t.C : t.O + 1);
   return size_t(words) * 8 + size_t(t.C) * elem;
 }
 
 template <bool HELD, typename Real>
 __device__ inline HeldTable hold_table(const MonomialTable& t, const int64_t* offsets, const Real* values,
                                        unsigned char* lds) {
-  if (!HELD) return {t.counts ? t.counts : t.ex, t.comp, t.toff, t.terms, t.outputs, offsets, values};
+  if (!HELD) return {nullptr, t.counts ? t.counts : t.ex, t.comp, t.toff, t.terms, t.outputs, offsets, values};
   auto copy = [&](const auto* from, int64_t n) {
     using T = std::remove_cv_t<std::remove_reference_t<decltype(*from)>>;
     T* to = reinterpret_cast<T*>(lds);
@@ -354,16 +357,49 @@ __device__ inline HeldTable hold_table(const MonomialTable& t, const int64_t* of
     h.toff = copy(t.toff, t.M + 1);
   }
   if (t.terms) h.terms = copy(t.terms, t.C);
+  if (t.counts && t.D <= kPackedComponents) {
+    // word M counts the monomials that do not fit, and the table is read as it is if any does not
+    uint64_t* const packed = reinterpret_cast<uint64_t*>(lds);
+    lds += size_t(t.M + 1) * 8;
+    if (threadIdx.x == 0) packed[t.M] = 0;
+    __syncthreads();
+    for (int64_t m = threadIdx.x; m < t.M; m += blockDim.x) {
+      uint64_t bits = 0;
+      bool fits = true;
+      for (int64_t c = 0; c < t.D; ++c) {
+        const int64_t e = t.counts[m * t.D + c];
+        fits = fits && e < 16;
+        bits |= uint64_t(e & 15) << (4 * c);
+      }
+      packed[m] = bits;
+      if (!fits) packed[t.M] = 1;
+    }
+    __syncthreads();
+    h.packed = packed[t.M] == 0 ? packed : nullptr;
+  }
   if (t.outputs) h.outputs = copy(t.outputs, t.C);
   if (offsets) h.offsets = copy(offsets, t.O + 1);
   h.values = copy(values, t.C);  // last: an odd number of 4-byte values would misalign what follows
   return h;
 }
 
-template <bool DENSE>
-__device__ inline void factor_range(const MonomialTable& t, const HeldTable& h, int64_t m, int64_t& q0, int64_t& q1) {
-  q0 = DENSE ? m * t.D : uniform64(h.toff[m]);
-  q1 = DENSE ? (m + 1) * t.D : uniform64(h.toff[m + 1]);
+// body(component, exponent) for each factor of monomial m that is not to the
+// power of zero.  A packed row is one read, and its zeros cost nothing.
+template <bool DENSE, typename Body>
+__device__ inline void for_factors(const MonomialTable& t, const HeldTable& h, int64_t m, Body body) {
+  if (DENSE && h.packed != nullptr) {
+    for (uint64_t bits = uint64_t(uniform64(int64_t(h.packed[m]))); bits != 0;) {
+      const int c = __builtin_ctzll(bits) >> 2;
+      body(c, int64_t(bits >> (4 * c)) & 15);
+      bits &= ~(uint64_t(15) << (4 * c));
+    }
+    return;
+  }
+  const int64_t q0 = DENSE ? m * t.D : uniform64(h.toff[m]), q1 = DENSE ? q0 + t.D : uniform64(h.toff[m + 1]);
+  for (int64_t q = q0; q < q1; ++q) {
+    const int64_t e = uniform64(h.exps[q]);
+    if (e != 0) body(int(DENSE ? q - q0 : uniform64(h.comp[q])), e);
+  }
 }
 
 // rows of x into xs[component][row]; rows past the batch hold ones
@@ -396,14 +432,8 @@ __global__ __launch_bounds__(512) void monomial_tile_kernel(const Real* __restri
     for (int64_t k = uniform64(h.offsets[o]); k < k1; ++k) {
       const Real v = uniform_value(hv[k]);
       const int64_t m = t.terms ? uniform64(h.terms[k]) : k;
-      int64_t q0, q1;
-      factor_range<DENSE>(t, h, m, q0, q1);
       Real p = t.terms ? Real(1) : v;
-      for (int64_t q = q0; q < q1; ++q) {
-        const int64_t e = uniform64(h.exps[q]);
-        if (e == 0) continue;
-        p *= ipow(xs[(DENSE ? q - q0 : uniform64(h.comp[q])) * kTileRows + lane], e);
-      }
+      for_factors<DENSE>(t, h, m, [&](int c, int64_t e) { p *= ipow(xs[c * kTileRows + lane], e); });
       if (t.terms) acc += v * p;
       else acc += p;
     }
@@ -457,16 +487,11 @@ __global__ __launch_bounds__(512) void monomial_tile_adjoint_kernel(
     if (o != before) g = gout[b * t.O + o];
     const Real v = uniform_value(hv[k]);
     const int64_t m = t.terms ? uniform64(h.terms[k]) : k;
-    int64_t q0, q1;
-    factor_range<DENSE>(t, h, m, q0, q1);
     const Real w = g * conjv(v);
     Real mono = Real(1);
     int64_t zdeg = 0;  // exponents of the zero factors (dense: those past one factor make it two or more)
-    int64_t zc = 0;
-    for (int64_t q = q0; q < q1; ++q) {
-      const int64_t e = uniform64(h.exps[q]);
-      if (e == 0) continue;
-      const int64_t c = DENSE ? q - q0 : uniform64(h.comp[q]);
+    int zc = 0;
+    for_factors<DENSE>(t, h, m, [&](int c, int64_t e) {
       const Real xv = xs[c * kTileRows + lane];
       if (xv == Real(0)) {
         zdeg += e;
@@ -474,14 +499,11 @@ __global__ __launch_bounds__(512) void monomial_tile_adjoint_kernel(
       } else {
         mono *= ipow(xv, e);
       }
-    }
+    });
     if (zdeg == 0) {
-      for (int64_t q = q0; q < q1; ++q) {
-        const int64_t e = uniform64(h.exps[q]);
-        if (e == 0) continue;
-        const int64_t c = DENSE ? q - q0 : uniform64(h.comp[q]);
+      for_factors<DENSE>(t, h, m, [&](int c, int64_t e) {
         grad[c * kTileRows + lane] += w * conjv(Real(e) * mono / xs[c * kTileRows + lane]);
-      }
+      });
     } else if (zdeg == 1) {
       grad[zc * kTileRows + lane] += w * conjv(mono);
     }
