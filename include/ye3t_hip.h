@@ -8,7 +8,8 @@
  *   - `dtype` is YE3T_F32 or YE3T_F64; float arrays of one call share it.
  *   - Work is enqueued on `stream` (NULL = default stream); calls never
  *     synchronise the device except plan creation, which copies tables, and
- *     ye3t_hip_check_indices, which waits for its answer.
+ *     ye3t_hip_check_indices and ye3t_hip_position_bounds, which wait for their
+ *     answers.
  *   - Return 0 on success, a negative ye3t_status on failure; the message of
  *     the last failure on the calling thread is ye3t_hip_last_error().
  *     Nothing throws across this boundary.
@@ -519,6 +520,11 @@ typedef struct {
   double cell_edge; /* >= cutoff * (1 + 1e-9) */
   int64_t dims[3];
 } ye3t_cell_grid;
+
+/* Smallest and largest coordinates of N >= 1 positions: bounds (host, 6 words)
+ * = min x, y, z, max x, y, z; an axis with a NaN coordinate has NaN for both.
+ * Waits for `stream`; YE3T_EUNSUPPORTED while it is captured. */
+int ye3t_hip_position_bounds(int dtype, const void* positions, int64_t N, double* bounds, ye3t_stream_t stream);
 
 /* Device workspace bytes of a neighbour-list build (-1 on invalid input). */
 int64_t ye3t_hip_neighbor_workspace_bytes(int64_t atom_count, const ye3t_cell_grid* grid);

@@ -128,6 +128,64 @@ int scan_inclusive(T* data, int64_t n, T* partials, hipStream_t s) {
   return check_launch("scan_add_kernel");
 }
 
+// ---- bounds ----------------------------------------------------------------
+
+// Each workgroup's smallest and largest coordinates, to host memory the device
+// can write: out[6 * block] = min x, y, z, max x, y, z; a NaN coordinate makes
+// its two NaN.  The host takes them together, so that the box is one kernel and one wait (a
+// reduction over the first axis, its conversions and two read-backs before:
+// 188 -> 155 us for a list of 50 000 atoms).
+constexpr int kBoundBlocks = 64;
+constexpr int kBoundThreads = 256;
+
+template <typename T>
+__global__ __launch_bounds__(kBoundThreads) void position_bounds_kernel(const T* __restrict__ pos, int64_t N,
+                                                                        double* __restrict__ out) {
+  __shared__ double part[kBoundThreads / 64][6];
+  double b[6];
+  auto lower = [](double a, double x) { return (x < a || x != x) ? x : a; };  // NaN stays: nothing is below it
+  auto upper = [](double a, double x) { return (x > a || x != x) ? x : a; };
+  const int64_t t = int64_t(blockIdx.x) * kBoundThreads + threadIdx.x;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) b[a] = b[3 + a] = double(pos[a]);
+  for (int64_t i = t; i < N; i += int64_t(gridDim.x) * kBoundThreads) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const double x = double(pos[3 * i + a]);
+      b[a] = lower(b[a], x);
+      b[3 + a] = upper(b[3 + a], x);
+    }
+  }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      b[a] = lower(b[a], __shfl_xor(b[a], d, 64));
+      b[3 + a] = upper(b[3 + a], __shfl_xor(b[3 + a], d, 64));
+    }
+  }
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int a = 0; a < 6; ++a) part[threadIdx.x >> 6][a] = b[a];
+  }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    const int a = threadIdx.x;
+    double v = part[0][a];
+    for (int w = 1; w < kBoundThreads / 64; ++w) v = a < 3 ? lower(v, part[w][a]) : upper(v, part[w][a]);
+    out[6 * blockIdx.x + a] = v;
+  }
+}
+
+// The calling thread's bounds: pinned host memory, made at its first list and
+// freed when the thread ends; a call waits for its kernel before it returns.
+struct BoundWords {
+  double* words = nullptr;
+  ~BoundWords() {
+    if (words != nullptr) (void)hipHostFree(words);
+  }
+};
+
 // ---- binning ---------------------------------------------------------------
 
 __global__ void clear_cells_kernel(int32_t* __restrict__ cell_start, int64_t cells, int64_t* __restrict__ row0) {
@@ -516,6 +574,44 @@ int fill_rows(int32_t N, const ye3t_cell_grid* grid, double cutoff, const Worksp
 using namespace ye3t;
 
 extern "C" {
+
+int ye3t_hip_position_bounds(int dtype, const void* positions, int64_t N, double* bounds, ye3t_stream_t stream) {
+  clear_error();
+  YE3T_REQUIRE(N >= 1 && positions && bounds, "bounds need positions and an output");
+  YE3T_REQUIRE(dtype == YE3T_F64 || dtype == YE3T_F32, "unsupported dtype %d", dtype);
+  const hipStream_t s = as_stream(stream);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  YE3T_CHECK_HIP(hipStreamIsCapturing(s, &capture));
+  if (capture != hipStreamCaptureStatusNone)
+    return set_error(YE3T_EUNSUPPORTED, "a neighbour list cannot be built while the stream is captured");
+  static thread_local BoundWords mine;
+  if (mine.words == nullptr) {
+    void* words = nullptr;
+    YE3T_CHECK_HIP(hipHostMalloc(&words, kBoundBlocks * 6 * sizeof(double), hipHostMallocPortable | hipHostMallocMapped));
+    mine.words = static_cast<double*>(words);
+  }
+  int64_t blocks = (N + kBoundThreads - 1) / kBoundThreads;
+  if (blocks > kBoundBlocks) blocks = kBoundBlocks;
+  if (dtype == YE3T_F64) {
+    hipLaunchKernelGGL(position_bounds_kernel<double>, dim3(unsigned(blocks)), dim3(kBoundThreads), 0, s,
+                       static_cast<const double*>(positions), N, mine.words);
+  } else {
+    hipLaunchKernelGGL(position_bounds_kernel<float>, dim3(unsigned(blocks)), dim3(kBoundThreads), 0, s,
+                       static_cast<const float*>(positions), N, mine.words);
+  }
+  const int rc = check_launch("position_bounds_kernel");
+  if (rc != YE3T_OK) return rc;
+  YE3T_CHECK_HIP(hipStreamSynchronize(s));
+  for (int a = 0; a < 6; ++a) {
+    double v = mine.words[a];
+    for (int64_t k = 1; k < blocks; ++k) {
+      const double x = mine.words[6 * k + a];
+      if (x != x || (a < 3 ? x < v : x > v)) v = x;
+    }
+    bounds[a] = v;
+  }
+  return YE3T_OK;
+}
 
 int64_t ye3t_hip_neighbor_workspace_bytes(int64_t atom_count, const ye3t_cell_grid* grid) {
   clear_error();

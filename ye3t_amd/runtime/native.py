@@ -191,6 +191,7 @@ def lib():
     L.ye3t_hip_factorized_angular_segmented_plan_info.argtypes = [_vp, _vp]
     L.ye3t_hip_factorized_angular_segmented_forward.argtypes = [_vp, _vp, _i64, _vp, _vp]
     L.ye3t_hip_factorized_angular_segmented_adjoint.argtypes = [_vp, _vp, _vp, _i64, _vp, _vp]
+    L.ye3t_hip_position_bounds.argtypes = [ctypes.c_int, _vp, _i64, ctypes.POINTER(ctypes.c_double), _vp]
     L.ye3t_hip_neighbor_workspace_bytes.argtypes = [_i64, ctypes.POINTER(CellGrid)]
     L.ye3t_hip_neighbor_workspace_bytes.restype = _i64
     L.ye3t_hip_neighbor_count.argtypes = [ctypes.c_int, _vp, _i64, ctypes.POINTER(CellGrid), ctypes.c_double, _vp,
@@ -232,7 +233,7 @@ EXPORTED_SYMBOLS = (
     "ye3t_hip_symmetric_power_shared_sparse_monomial_adjoint",
     "ye3t_hip_symmetric_power_shared_sparse_monomial_double_backward", "ye3t_hip_code_object_kernel_info",
     "ye3t_hip_part_private_limit", "ye3t_hip_check_indices",
-    "ye3t_hip_csr_offsets",
+    "ye3t_hip_csr_offsets", "ye3t_hip_position_bounds",
 )
 
 
@@ -1552,8 +1553,10 @@ def neighbor_list(positions, cutoff, grid=None):
     dev = positions.device
     if grid is None:
         if N:
-            lo, hi = torch.aminmax(positions, dim=0)
-            lo, hi = lo.double().cpu().tolist(), hi.double().cpu().tolist()
+            bounds = (ctypes.c_double * 6)()
+            _check(lib().ye3t_hip_position_bounds(_dtype_code(positions), _dev(positions, "positions"), N, bounds,
+                                                  _stream()), "ye3t_hip_position_bounds")
+            lo, hi = list(bounds[:3]), list(bounds[3:])
         else:
             lo = hi = [0.0, 0.0, 0.0]
         grid = cell_grid(lo, hi, cutoff, N)
