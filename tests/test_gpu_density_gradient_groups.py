@@ -39,3 +39,28 @@ def test_grouped_edge_gradient(gpu, mode, channels, atoms, degree, n_max, l_max,
     assert inp["edge_count"] >= 65536
     flush(f"  {err:.2e}")
     assert err < (TOL["f64"] if dtype == "f64" else TOL["f32"])
+
+
+@pytest.mark.parametrize("mode,channels,dtypes", [("single", 1, ("f64", "f64")), ("species", 3, ("f32", "f64"))])
+@pytest.mark.parametrize("n_max", [0, 1])
+@pytest.mark.parametrize("lam", [0.0, 800.0])
+def test_rows_that_lambda_does_not_enter(gpu, mode, channels, dtypes, n_max, lam):
+    """R_0 and R_1 hold no lambda: where expm1(lambda) is zero or infinite, and higher rows are no numbers,
+    a model of those two rows has the gradient it always had."""
+    flush(f"grouped edge gradient {mode} x{channels}, n_max {n_max}, lambda {lam}, {dtypes}")
+    import torch
+
+    from ye3t_amd.runtime import native
+
+    inp = _workload(mode, 1500, 100, 93, n_max, 4, channels)
+    inp["lambda"] = lam
+    gA = np.random.default_rng(94).normal(size=(1500, channels, n_max + 1, 25))
+    d, kw = _device(inp, dtypes[0], gpu)
+    gd = torch.as_tensor(gA, device=gpu)
+    got = native.ace_density_edge_gradient(gd, d["edge_vectors"], d["row_offsets"], d["neighbors"], **kw)
+    ref = oracle.ace_density_edge_gradient(rounded_inputs(inp, dtypes[0]), gA)
+    assert inp["edge_count"] >= 65536
+    got = got.cpu().numpy()
+    err = max(column_rel_error(got, ref), column_rel_error(got[3:], ref[3:]))
+    flush(f"  {err:.2e}")
+    assert np.isfinite(ref).all() and err < TOL[dtypes[0]]

@@ -272,7 +272,7 @@ __device__ inline void gm_radial(double r, const GmRadial& c, double (&R)[NRC], 
 // groups whose adjoint blocks are on their way at once
 constexpr int kGmAhead = 4;
 
-// NRC: radial rows compiled (>= p.nr; rows from p.nr on meet a zero adjoint).
+// NRC: radial rows compiled (>= p.nr; rows from p.nr on are not read).
 template <int LMAX, int NRC, typename In, typename G>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, LMAX >= 6 ? 1 : 2))) void
 density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, int64_t waves) {
@@ -351,7 +351,9 @@ density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, int64_t 
       for (int ct = 0; ct < CT; ++ct) t[ct] = u[ct] = 0.0;
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        const int n = 4 * s + kq < NRC ? 4 * s + kq : NRC - 1;
+        // rows past the model's last meet a zero adjoint, but may hold no number themselves (0 / 0 at
+        // lambda 0, where rows 0 and 1 are well defined): the last row stands in for them
+        const int n = 4 * s + kq < p.nr ? 4 * s + kq : p.nr - 1;
         const double ar = At[n][ci], ad = At[NRC + n][ci];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
