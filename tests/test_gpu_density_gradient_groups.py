@@ -64,3 +64,34 @@ def test_rows_that_lambda_does_not_enter(gpu, mode, channels, dtypes, n_max, lam
     err = max(column_rel_error(got, ref), column_rel_error(got[3:], ref[3:]))
     flush(f"  {err:.2e}")
     assert np.isfinite(ref).all() and err < TOL[dtypes[0]]
+
+
+@pytest.mark.parametrize("mode,channels", [("single", 1), ("species", 3)])
+@pytest.mark.parametrize("degrees", ["one atom", "first tenth", "last atoms", "far apart", "few atoms", "rising"])
+def test_uneven_structures(gpu, mode, channels, degrees):
+    """Shares of the work that begin and end within atoms, runs of empty atoms longer than a chunk's window at
+    the start, between and at the end, and atoms of many chunks."""
+    flush(f"grouped edge gradient {mode} x{channels}, {degrees}")
+    import torch
+
+    from ye3t_amd.runtime import native
+
+    rng = np.random.default_rng(95)
+    counts = {"one atom": [70001], "first tenth": [230] * 300 + [0] * 2700, "last atoms": [0] * 5000 + [337] * 201,
+              "far apart": np.where(np.arange(5000) % 76 == 7, 1009, 0), "few atoms": [701] * 97,
+              "rising": np.arange(1500) // 16}[degrees]
+    inp = _workload(mode, len(counts), 1, 96, 6, 4, channels)
+    E = int(np.sum(counts))
+    vec = rng.normal(size=(E, 3))
+    inp.update(edge_count=E, centers=np.repeat(np.arange(len(counts)), counts),
+               row_offsets=np.concatenate([[0], np.cumsum(counts)]).astype(np.int64),
+               neighbors=rng.integers(0, len(counts), E),
+               edge_vectors=vec / np.linalg.norm(vec, axis=1, keepdims=True) * rng.uniform(0.05, 5.3, (E, 1)))
+    gA = rng.normal(size=(len(counts), channels, 7, 25))
+    d, kw = _device(inp, "f64", gpu)
+    got = native.ace_density_edge_gradient(torch.as_tensor(gA, device=gpu), d["edge_vectors"], d["row_offsets"],
+                                           d["neighbors"], **kw)
+    assert E >= 65536
+    err = column_rel_error(got.cpu().numpy(), oracle.ace_density_edge_gradient(inp, gA))
+    flush(f"  {err:.2e}")
+    assert err < TOL["f64"]

@@ -8,8 +8,9 @@
 // are products of an [edges x n] by an [n x k] matrix that all edges of one
 // (atom, channel) group share.  The lane-per-edge kernel gathers the block once
 // per edge: 637 loads an edge at n_max 12, l_max 6, from as many cache lines as
-// a wave has groups.  Here one wave walks its atoms in chunks of whole atoms
-// with at most 64 edges together:
+// a wave has groups.  Here one wave walks an equal share of the edges in chunks
+// of whole atoms with at most 64 edges together (a share or an atom of more
+// edges may end a chunk within an atom, whose groups are then read twice):
 //   basis    lane = edge: radial values and derivatives and harmonics, to LDS
 //            at the edge's column, columns grouped by (atom, channel);
 //   product  per group; the block comes straight from global memory in the
@@ -80,8 +81,8 @@ __device__ inline G gm_load(__amdgpu_buffer_rsrc_t rb, unsigned voff, unsigned s
 __device__ inline int64_t gm_clamp(int64_t i, int64_t n) { return i < 0 ? 0 : (i >= n ? n - 1 : i); }
 
 // Up to 64 whole atoms with at most 64 edges together from edge e of atom a on,
-// or 64 edges of an atom that has more of them left.  `end` of lane j is the
-// end of atom a + j relative to e.
+// or 64 edges of an atom that has more of them left, of the edges before the
+// wave's end.  `end` of lane j is the end of atom a + j relative to e.
 struct GmChunk {
   int64_t a, e;
   int na, cnt;
@@ -90,23 +91,98 @@ struct GmChunk {
 
 // offsets of the atoms after a, one per lane
 template <typename In, typename G>
-__device__ inline int64_t gm_window(const GradParams<In, G>& p, int64_t a, int64_t a_end, int lane) {
-  return p.row_offsets[a + 1 + lane < a_end ? a + 1 + lane : a_end];
+__device__ inline int64_t gm_window(const GradParams<In, G>& p, int64_t a, int lane) {
+  return p.row_offsets[a + 1 + lane < p.N ? a + 1 + lane : p.N];
 }
 
-__device__ inline GmChunk gm_form(int64_t a, int64_t e, int64_t a_end, int64_t window, int64_t edges, int lane) {
+// lane 0's value
+__device__ inline int64_t gm_first(int64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(int(uint32_t(uint64_t(v))));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(int(uint32_t(uint64_t(v) >> 32)));
+  return int64_t((uint64_t(hi) << 32) | lo);
+}
+
+// For each of `key`, the last atom i with row_offsets[i] + per_atom * i <= key
+// (atom 0 if there is none): 64 probes a step for all of them, three steps up
+// to 262 144 atoms.
+template <int K, typename In, typename G>
+__device__ inline void gm_atoms(const GradParams<In, G>& p, const int64_t (&key)[K], int64_t per_atom, int lane,
+                                int64_t (&lo)[K]) {
+  int64_t n[K];
+  bool more = false;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    lo[k] = 0;
+    n[k] = p.N;
+    more = more || n[k] > 1;
+  }
+  while (more) {
+    more = false;
+    int64_t at[K], off[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      at[k] = lane * ((n[k] + 63) >> 6);
+      at[k] = at[k] < n[k] ? at[k] : 0;
+      off[k] = p.row_offsets[lo[k] + at[k]];
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int64_t step = (n[k] + 63) >> 6;
+      const uint64_t m = gm_ballot(lane == 0 || (at[k] > 0 && off[k] + per_atom * (lo[k] + at[k]) <= key[k]));
+      const int hit = ~m == 0 ? 63 : __builtin_ctzll(~m) - 1;  // the keys rise: the probes that pass are a prefix
+      lo[k] += hit * step;
+      n[k] -= hit * step;
+      n[k] = n[k] < step ? n[k] : step;
+      more = more || n[k] > 1;
+    }
+  }
+}
+
+// A share of the work ends, and the next begins, at `key` in atom a (whose
+// edges start at `first` and end at `last`): an atom's work is its edges and,
+// for the quads that its groups fill in part, `per_atom` edges more.  Atoms of at
+// most 64 edges are not cut: their chunks would be more, not shorter.
+__device__ inline int64_t gm_bound(int64_t key, int64_t per_atom, int64_t a, int64_t first, int64_t last, int64_t edges) {
+  first = gm_clamp(first, edges + 1);
+  last = gm_clamp(last, edges + 1);
+  const int64_t in = key - per_atom * (a + 1) - first;
+  return last - first <= 64 || in < 0 ? first : first + (in & ~int64_t(3));
+}
+
+// The chunk at (a, e), from the offsets `window` after a.  The wave's last
+// edge ends its last atom, and the last atom ends the edges.
+template <typename In, typename G>
+__device__ inline GmChunk gm_take(const GradParams<In, G>& p, int64_t a, int64_t e, int64_t e_end, int64_t window,
+                                  int lane) {
   GmChunk c;
   c.a = a;
   c.e = e;
-  const int64_t rel = gm_clamp(window, edges + 1) - e;  // offsets clamped into the edge array
+  const int left = e_end - e < 65 ? int(e_end - e) : 65;
+  const int64_t rel = (a + 1 + lane < p.N && window < e_end ? window : e_end) - e;
   c.end = rel < 0 ? 0 : (rel > 65 ? 65 : int(rel));
-  const uint64_t fits = gm_ballot(a + 1 + lane <= a_end && c.end <= 64);
-  // the fitting atoms are a prefix (the offsets rise)
-  c.na = ~fits == 0 ? 64 : __builtin_ctzll(~fits);
-  if (c.na > 0) {
-    c.cnt = __builtin_amdgcn_readlane(c.end, c.na - 1);
-  } else {
-    c.cnt = a < a_end ? 64 : 0;
+  const uint64_t fits = gm_ballot(a + 1 + lane <= p.N && c.end <= 64);
+  const uint64_t before = gm_ballot(c.end < left);
+  // both are prefixes (the offsets rise); the atom after those that end before the wave does is its last
+  const int nf = ~fits == 0 ? 64 : __builtin_ctzll(~fits);
+  const int nb = ~before == 0 ? 64 : __builtin_ctzll(~before) + 1;
+  c.na = left <= 0 ? 0 : (nf < nb ? nf : nb);
+  c.cnt = c.na > 0 ? __builtin_amdgcn_readlane(c.end, c.na - 1) : (left <= 0 ? 0 : (left < 64 ? left : 64));
+  return c;
+}
+
+template <typename In, typename G>
+__device__ inline GmChunk gm_form(const GradParams<In, G>& p, int64_t a, int64_t e, int64_t e_end, int64_t window,
+                                  int lane) {
+  GmChunk c = gm_take(p, a < p.N ? a : p.N - 1, e, e_end, window, lane);
+  if (c.cnt == 0 && e < e_end) {  // empty atoms only: on to the atom that holds edge e
+    int64_t to[1];
+    gm_atoms<1>(p, {e}, 0, lane, to);
+    a = to[0];
+    c = gm_take(p, a, e, e_end, gm_window(p, a, lane), lane);
+    if (c.cnt == 0) {  // offsets that fall: the edges are this atom's, so that the wave ends
+      c.na = 0;
+      c.cnt = e_end - e < 64 ? int(e_end - e) : 64;
+    }
   }
   return c;
 }
@@ -269,13 +345,20 @@ __device__ inline void gm_radial(double r, const GmRadial& c, double (&R)[NRC], 
   }
 }
 
+// Shares of a launch: the work is the edges and `per_atom` for each atom (a
+// group leaves one and a half of a quad's four places empty on average), the
+// first `larger` waves have size + 1 of it and the others size.
+struct GmShares {
+  int64_t size, larger, per_atom;
+};
+
 // groups whose adjoint blocks are on their way at once
 constexpr int kGmAhead = 4;
 
 // NRC: radial rows compiled (>= p.nr; rows from p.nr on are not read).
 template <int LMAX, int NRC, typename In, typename G>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, LMAX >= 6 ? 1 : 2))) void
-density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, int64_t waves) {
+density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, GmShares shares) {
   constexpr int LW = (LMAX + 1) * (LMAX + 1);
   constexpr int CT = (LW + 15) / 16;
   constexpr int KS = (NRC + 3) / 4;        // k-steps of four
@@ -287,9 +370,19 @@ density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, int64_t 
   const int lane = threadIdx.x;
   const int kq = lane >> 4, cc = lane & 15;
   const uint64_t lt = (uint64_t(1) << lane) - 1;
-  const int64_t a_begin = int64_t(blockIdx.x) * p.N / waves;
-  const int64_t a_end = (int64_t(blockIdx.x) + 1) * p.N / waves;
-  if (a_begin >= a_end) return;
+  const int64_t share = int64_t(blockIdx.x);
+  const int64_t keys[2] = {shares.size * share + (share < shares.larger ? share : shares.larger),
+                           shares.size * (share + 1) + (share + 1 < shares.larger ? share + 1 : shares.larger)};
+  int64_t atoms[2];
+  gm_atoms<2>(p, keys, shares.per_atom, lane, atoms);
+  const int64_t first = p.row_offsets[atoms[0]], first_after = p.row_offsets[atoms[1]];
+  const int64_t last_after = p.row_offsets[atoms[1] + 1];
+  int64_t window = gm_window(p, atoms[0], lane);
+  const int64_t e_begin = share == 0 ? 0 : gm_bound(keys[0], shares.per_atom, atoms[0], first, gm_first(window), p.E);
+  const int64_t e_end = share + 1 == int64_t(gridDim.x)
+                            ? p.E
+                            : gm_bound(keys[1], shares.per_atom, atoms[1], first_after, last_after, p.E);
+  if (e_begin >= e_end) return;
   const int64_t block = int64_t(p.nr) * LW;
   const unsigned voff = unsigned(kq * LW + cc) * unsigned(sizeof(G));
   auto channel = [&](const GmEdge<In>& edge) {
@@ -383,13 +476,11 @@ density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, int64_t 
   // chunk i + 1, which then have the chain of chunk i and the basis of chunk
   // i + 1 to arrive in.  The species of chunk i + 1 are gathered during the
   // basis and products of chunk i.
-  int64_t e0 = p.row_offsets[a_begin];
-  e0 = gm_clamp(e0, p.E + 1);
-  GmChunk cur = gm_form(a_begin, e0, a_end, gm_window(p, a_begin, a_end, lane), p.E, lane);
+  GmChunk cur = gm_form(p, atoms[0], e_begin, e_end, window, lane);
   GmEdge<In> E = gm_edge(p, cur, lane);
-  GmChunk nxt = gm_form(cur.a + cur.na, cur.e + cur.cnt, a_end, gm_window(p, cur.a + cur.na, a_end, lane), p.E, lane);
+  GmChunk nxt = gm_form(p, cur.a + cur.na, cur.e + cur.cnt, e_end, gm_window(p, cur.a + cur.na, lane), lane);
   GmEdge<In> NE = gm_edge(p, nxt, lane);
-  int64_t window = gm_window(p, nxt.a + nxt.na, a_end, lane);
+  window = gm_window(p, nxt.a + nxt.na, lane);
   int col = 0, ng = 0;
   int3 g[kGmAhead];
   G b[kGmAhead][KS][CT];
@@ -399,7 +490,7 @@ density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, int64_t 
     g[d] = entry(d);
     fetch(cur.a, d < ng, g[d], b[d]);
   }
-  while (cur.a < a_end) {
+  while (cur.e < e_end) {
     const bool valid = lane < cur.cnt;
     const int nsp = channel(NE);
     const double vx = double(E.x), vy = double(E.y), vz = double(E.z);
@@ -438,9 +529,9 @@ density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, int64_t 
     // ---- the chunk after next, and the next one's groups and first blocks
     const int tcol = col;
     group(nxt, nsp, col, ng);
-    const GmChunk nn = gm_form(nxt.a + nxt.na, nxt.e + nxt.cnt, a_end, window, p.E, lane);
+    const GmChunk nn = gm_form(p, nxt.a + nxt.na, nxt.e + nxt.cnt, e_end, window, lane);
     const GmEdge<In> NNE = gm_edge(p, nn, lane);
-    window = gm_window(p, nn.a + nn.na, a_end, lane);
+    window = gm_window(p, nn.a + nn.na, lane);
 #pragma unroll
     for (int d = 0; d < kGmAhead; ++d) {
       g[d] = entry(d);
@@ -487,9 +578,13 @@ int launch_shape(const GradParams<In, G>& p, hipStream_t s) {
   radial.lambda = p.lambda;
   radial.den = std::expm1(p.lambda);
   int64_t waves = int64_t(cus) * per_cu;  // as many as the device holds at once
-  if (waves > p.N) waves = p.N;
+  if (waves > (p.E + 63) / 64) waves = (p.E + 63) / 64;
+  GmShares shares;
+  shares.per_atom = (3 * int64_t(p.C) + 1) / 2;
+  shares.size = (p.E + shares.per_atom * p.N) / waves;
+  shares.larger = (p.E + shares.per_atom * p.N) % waves;
   hipLaunchKernelGGL((density_edge_gradient_mfma_kernel<LMAX, NRC, In, G>), dim3(unsigned(waves)),
-                     dim3(64), 0, s, p, radial, waves);
+                     dim3(64), 0, s, p, radial, shares);
   return check_launch("density_edge_gradient_mfma_kernel");
 }
 
@@ -503,12 +598,15 @@ int launch_lmax(const GradParams<In, G>& p, hipStream_t s) {
 
 }  // namespace
 
-// Taken where a group fills its four rows on average and the launch fills the
-// chip.  Both sides measured (lane-per-edge / here, us): at 20 000 atoms x 32,
-// l_max 4, n_max 8, ten edges a group 110 / 84 and four 137 / 135; l_max 6,
-// n_max 12, 282 / 158 and 330 / 257; below four edges a group (5 000 x 16,
+// Taken where a group fills its four rows on average and there are edges for
+// every wave.  Both sides measured (lane-per-edge / here, us): at 20 000 atoms
+// x 32, l_max 4, n_max 10, one channel 95 / 76 and four 121 / 98; l_max 6,
+// n_max 12, 182 / 131 and 295 / 185; below four edges a group (5 000 x 16,
 // 8 species, l_max 4) 28 / 35; below l_max 4 the blocks are small enough for
 // the lane-per-edge kernel (l_max 2: 33 / 71; l_max 3: 62 / 51 to 111 / 116).
+// Uneven structures at n_max 10, l_max 4, four species: all edges in a tenth of
+// 20 000 atoms 141 / 98, degrees rising from 0 to 64 147 / 117, 100 atoms x 700
+// 20 / 19 (551, 132 and 90 with equal shares of the atoms).
 template <typename In, typename G>
 int launch_edge_gradient_mfma(const GradParams<In, G>& p, int lmax, hipStream_t s) {
   if (p.mix || p.feats || p.C > (1 << 24)) return YE3T_EUNSUPPORTED;  // a group's block is 32-bit within its chunk
