@@ -41,6 +41,12 @@ def test_grouped_edge_gradient(gpu, mode, channels, atoms, degree, n_max, l_max,
     assert err < (TOL["f64"] if dtype == "f64" else TOL["f32"])
 
 
+def _error(got, ref):
+    """The three edges below epsilon are larger than the others by their 1 / epsilon, and a root mean square over
+    all E edges is sqrt(E / 3) below theirs: each part by itself."""
+    return max(column_rel_error(got[:3], ref[:3]), column_rel_error(got[3:], ref[3:]))
+
+
 @pytest.mark.parametrize("mode,channels,dtypes", [("single", 1, ("f64", "f64")), ("species", 3, ("f32", "f64"))])
 @pytest.mark.parametrize("n_max", [0, 1])
 @pytest.mark.parametrize("lam", [0.0, 800.0])
@@ -61,7 +67,7 @@ def test_rows_that_lambda_does_not_enter(gpu, mode, channels, dtypes, n_max, lam
     ref = oracle.ace_density_edge_gradient(rounded_inputs(inp, dtypes[0]), gA)
     assert inp["edge_count"] >= 65536
     got = got.cpu().numpy()
-    err = max(column_rel_error(got, ref), column_rel_error(got[3:], ref[3:]))
+    err = _error(got, ref)
     flush(f"  {err:.2e}")
     assert np.isfinite(ref).all() and err < TOL[dtypes[0]]
 
@@ -77,21 +83,43 @@ def test_uneven_structures(gpu, mode, channels, degrees):
     from ye3t_amd.runtime import native
 
     rng = np.random.default_rng(95)
-    counts = {"one atom": [70001], "first tenth": [230] * 300 + [0] * 2700, "last atoms": [0] * 5000 + [337] * 201,
-              "far apart": np.where(np.arange(5000) % 76 == 7, 1009, 0), "few atoms": [701] * 97,
-              "rising": np.arange(1500) // 16}[degrees]
-    inp = _workload(mode, len(counts), 1, 96, 6, 4, channels)
+    counts = {"one atom": [100003], "first tenth": [230] * 450 + [0] * 4050, "last atoms": [0] * 5000 + [337] * 297,
+              "far apart": np.where(np.arange(5000) % 50 == 7, 1009, 0), "few atoms": [701] * 143,
+              "rising": np.arange(1800) // 16}[degrees]
+    inp = _workload(mode, len(counts), 1, 96, 15, 6, channels)
     E = int(np.sum(counts))
     vec = rng.normal(size=(E, 3))
     inp.update(edge_count=E, centers=np.repeat(np.arange(len(counts)), counts),
                row_offsets=np.concatenate([[0], np.cumsum(counts)]).astype(np.int64),
                neighbors=rng.integers(0, len(counts), E),
                edge_vectors=vec / np.linalg.norm(vec, axis=1, keepdims=True) * rng.uniform(0.05, 5.3, (E, 1)))
-    gA = rng.normal(size=(len(counts), channels, 7, 25))
+    gA = rng.normal(size=(len(counts), channels, 16, 49))
     d, kw = _device(inp, "f64", gpu)
     got = native.ace_density_edge_gradient(torch.as_tensor(gA, device=gpu), d["edge_vectors"], d["row_offsets"],
                                            d["neighbors"], **kw)
-    assert E >= 65536
+    assert E * 16 * 49 >= 7.5e7 and E // 4 >= len(counts) * channels
     err = column_rel_error(got.cpu().numpy(), oracle.ace_density_edge_gradient(inp, gA))
     flush(f"  {err:.2e}")
     assert err < TOL["f64"]
+
+
+@pytest.mark.parametrize("channels,dtypes", [(1, ("f64", "f64")), (3, ("f32", "f64")), (2, ("f32", "f32"))])
+@pytest.mark.parametrize("n_max", [6, 7, 8, 10, 11, 12, 13, 15])
+def test_radial_rows(gpu, n_max, channels, dtypes):
+    """Every count of compiled radial rows, filled and in part."""
+    flush(f"grouped edge gradient, {channels} channels, n_max {n_max}, {dtypes}")
+    import torch
+
+    from ye3t_amd.runtime import native
+
+    inp = _workload("species" if channels > 1 else "single", 4500 if channels == 1 else 1500, 100, 97, n_max, 6, channels)
+    shape = (inp["atom_count"], channels, n_max + 1, 49)
+    assert inp["edge_count"] * (n_max + 1) * 49 >= (7.5e7 if channels == 1 else 2.5e7)
+    d, kw = _device(inp, dtypes[0], gpu)
+    gd = torch.as_tensor(np.random.default_rng(98).normal(size=shape), device=gpu)
+    gd = gd.to(torch.float64 if dtypes[1] == "f64" else torch.float32)
+    got = native.ace_density_edge_gradient(gd, d["edge_vectors"], d["row_offsets"], d["neighbors"], **kw).cpu().numpy()
+    ref = oracle.ace_density_edge_gradient(rounded_inputs(inp, dtypes[0]), gd.double().cpu().numpy())
+    err = _error(got, ref)
+    flush(f"  {err:.2e}")
+    assert err < TOL[dtypes[0]]

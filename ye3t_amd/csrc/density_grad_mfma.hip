@@ -20,9 +20,9 @@
 //            to the sixteen of the larger shape (its average is six at eight
 //            species and 48 neighbours); t replaces Y in LDS;
 //   chain    lane = edge: the gradient of the harmonics contracted with t.
-// Measured (kernel trace): 8 species, n_max 12, l_max 6, 30 000 atoms x 48:
-// 731 us for the lane-per-edge kernel, 480 us here; 4 species, n_max 10,
-// l_max 4, 20 000 x 32: 158 and 106 us.  It is bound by one wave per SIMD
+// Measured (events): 8 species, n_max 12, l_max 6, 30 000 atoms x 48: 691 us for
+// the lane-per-edge kernel, 470 us here; 4 species, n_max 10, l_max 4,
+// 20 000 x 32: 121 and 100 us.  It is bound by one wave per SIMD
 // (two at l_max 4) working through dependent fp64 instructions: the tile, 40 KB
 // at l_max 6, limits how many are resident.  Without the block loads it takes
 // 469 us, without the products 161.  Four waves sharing a tile, each with a
@@ -352,12 +352,15 @@ struct GmShares {
   int64_t size, larger, per_atom;
 };
 
+// waves a SIMD that a kernel is compiled for
+constexpr int kGmSimdWaves(int lmax) { return lmax >= 6 ? 1 : 2; }
+
 // groups whose adjoint blocks are on their way at once
 constexpr int kGmAhead = 4;
 
 // NRC: radial rows compiled (>= p.nr; rows from p.nr on are not read).
 template <int LMAX, int NRC, typename In, typename G>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, LMAX >= 6 ? 1 : 2))) void
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, kGmSimdWaves(LMAX)))) void
 density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, GmShares shares) {
   constexpr int LW = (LMAX + 1) * (LMAX + 1);
   constexpr int CT = (LW + 15) / 16;
@@ -562,17 +565,35 @@ density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, GmShares
   }
 }
 
+// Waves of a compute unit: as many as its LDS holds tiles (allocated in steps of
+// 1 280 bytes) and its SIMDs waves of the kernel, but not five, of which two
+// share a SIMD while three have their own: the launch ends with that pair (l_max
+// 5, n_max 7: 92 us, with four 88).
+template <int LMAX, int NRC, typename In, typename G>
+int gm_waves() {
+  int regs = 0, lds = 0;
+  hipFuncAttributes at;
+  if (hipFuncGetAttributes(&at, reinterpret_cast<const void*>(&density_edge_gradient_mfma_kernel<LMAX, NRC, In, G>)) ==
+      hipSuccess) {
+    regs = at.numRegs;
+    lds = int(at.sharedSizeBytes);
+  } else {
+    (void)hipGetLastError();
+  }
+  if (lds <= 0) return 4;
+  const int tiles = 160 * 1024 / ((lds + 1279) / 1280 * 1280);
+  const int simd = regs > 256 ? 1 : kGmSimdWaves(LMAX);
+  const int waves = tiles < 4 * simd ? tiles : 4 * simd;
+  return waves == 5 ? 4 : waves;
+}
+
 template <int LMAX, int NRC, typename In, typename G>
 int launch_shape(const GradParams<In, G>& p, hipStream_t s) {
-  auto* const kernel = &density_edge_gradient_mfma_kernel<LMAX, NRC, In, G>;
-  int dev = 0, cus = 0, per_cu = 0;
+  static const int per_cu = gm_waves<LMAX, NRC, In, G>();  // the kernel's own, the same on every gfx950
+  int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
     cus = 256;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel),
-                                                   64, 0) != hipSuccess ||
-      per_cu <= 0)
-    per_cu = 4;
   GmRadial radial;
   radial.rc = p.cutoff > 2.220446049250313e-16 ? p.cutoff : 2.220446049250313e-16;
   radial.lambda = p.lambda;
@@ -588,29 +609,45 @@ int launch_shape(const GradParams<In, G>& p, hipStream_t s) {
   return check_launch("density_edge_gradient_mfma_kernel");
 }
 
+// Rows compiled: whole steps of four (8, 12, 16), and below 12 and 16 the most
+// whose tile leaves room for another wave in a compute unit (11: six rather than
+// five at l_max 4; 13: four rather than three at l_max 6).
 template <int LMAX, typename In, typename G>
 int launch_lmax(const GradParams<In, G>& p, hipStream_t s) {
-  if (p.nr <= 9) return launch_shape<LMAX, 9>(p, s);
+  if (p.nr <= 8) return launch_shape<LMAX, 8>(p, s);
   if (p.nr <= 11) return launch_shape<LMAX, 11>(p, s);
+  if (p.nr <= 12) return launch_shape<LMAX, 12>(p, s);
   if (p.nr <= 13) return launch_shape<LMAX, 13>(p, s);
   return launch_shape<LMAX, 16>(p, s);
 }
 
 }  // namespace
 
-// Taken where a group fills its four rows on average and there are edges for
-// every wave.  Both sides measured (lane-per-edge / here, us): at 20 000 atoms
-// x 32, l_max 4, n_max 10, one channel 95 / 76 and four 121 / 98; l_max 6,
-// n_max 12, 182 / 131 and 295 / 185; below four edges a group (5 000 x 16,
-// 8 species, l_max 4) 28 / 35; below l_max 4 the blocks are small enough for
-// the lane-per-edge kernel (l_max 2: 33 / 71; l_max 3: 62 / 51 to 111 / 116).
+// Taken where a group fills its four rows on average, where the radial rows
+// fill two steps of four, and where the other kernel's gathers (E nr (l_max +
+// 1)^2 values) cost more than the start of a wave here: 2.5e7 of them, three
+// times as many with one channel, whose edges gather the same block together.
+// Both sides measured (lane-per-edge / here, us):
+//   edges a group   5 000 x 16, 8 species, l_max 4 (two): 28 / 35; 20 000 x 32,
+//                   l_max 4, 4 species (eight), n_max 10: 121 / 98
+//   radial rows     400 000 edges, 4 species, n_max 1, 3, 5, 7, 10, 15:
+//                   l_max 4: 38 / 43, 47 / 44, 58 / 52, 67 / 51, 82 / 68, 133 / 84
+//                   l_max 5: 45 / 60, 67 / 60, 70 / 79, 102 / 80, 98 / 88, 175 / 101
+//                   l_max 6: 60 / 76, 77 / 76, 93 / 87, 113 / 88, 142 / 104, 267 / 169
+//   gathers         n_max 7, 4 species, l_max 4, 66 000 and 132 000 edges (1.3e7,
+//                   2.6e7): 16 / 17, 28 / 26; l_max 6 (2.6e7, 5.2e7): 31 / 26,
+//                   49 / 39; one channel, n_max 10, l_max 4, 132 000, 264 000,
+//                   400 000 edges (3.6e7, 7.3e7, 1.1e8): 24 / 24, 45 / 38, 66 / 55
+//   l_max           below 4 the blocks are small enough for the lane-per-edge
+//                   kernel (l_max 2: 33 / 71; l_max 3: 62 / 51 to 111 / 116)
 // Uneven structures at n_max 10, l_max 4, four species: all edges in a tenth of
-// 20 000 atoms 141 / 98, degrees rising from 0 to 64 147 / 117, 100 atoms x 700
-// 20 / 19 (551, 132 and 90 with equal shares of the atoms).
+// 20 000 atoms 141 / 98, degrees rising from 0 to 64 147 / 117 (551 and 132 with
+// equal shares of the atoms).
 template <typename In, typename G>
 int launch_edge_gradient_mfma(const GradParams<In, G>& p, int lmax, hipStream_t s) {
   if (p.mix || p.feats || p.C > (1 << 24)) return YE3T_EUNSUPPORTED;  // a group's block is 32-bit within its chunk
-  if (p.E < 65536 || p.E / 4 < p.N * int64_t(p.C)) return YE3T_EUNSUPPORTED;
+  if (p.E < 65536 || p.E / 4 < p.N * int64_t(p.C) || p.nr < 7) return YE3T_EUNSUPPORTED;
+  if (double(p.E) * (p.nr * (lmax + 1) * (lmax + 1)) < (p.C > 1 ? 2.5e7 : 7.5e7)) return YE3T_EUNSUPPORTED;
   switch (lmax) {
     case 4: return launch_lmax<4>(p, s);
     case 5: return launch_lmax<5>(p, s);
