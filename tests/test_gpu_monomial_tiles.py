@@ -73,3 +73,22 @@ def test_complex_supports_equal_a_real_pair(gpu, rows):
     assert torch.allclose(out, 1j * real.forward(x), rtol=1e-14, atol=1e-14)
     grad = turned.adjoint(g.to(torch.complex128), x.to(torch.complex128))
     assert torch.allclose(grad, -1j * real.adjoint(g, x), rtol=1e-13, atol=1e-13)
+
+
+@pytest.mark.parametrize("dtype,big", [("f32", 1e10), ("f64", 1e75)])
+def test_grouped_values_scale_their_monomials(gpu, dtype, big):
+    """A value that brings a product into range, which the bare product leaves: forward and gradient start from
+    the value."""
+    flush(f"grouped monomials in range by their values, {dtype}")
+    import torch
+
+    from ye3t_amd import runtime
+
+    real = torch.float64 if dtype == "f64" else torch.float32
+    counts, vals = np.array([[3, 2], [0, 3]]), np.array([big ** -2, -(big ** -1)])
+    x = torch.tensor([[big, -2 * big]] * 3, dtype=real, device=gpu, requires_grad=True)
+    out = runtime.symmetric_power_monomial_contraction(x, counts, np.array([0, 1, 2]), np.array([0, 1]), vals)
+    (gx,) = torch.autograd.grad(out, x, torch.ones_like(out))
+    want = [12 * big ** 2, -4 * big ** 2 - 12 * big]
+    assert torch.allclose(gx.double(), torch.tensor([want] * 3, device=gpu, dtype=torch.float64),
+                          rtol=1e-14 if dtype == "f64" else 1e-6, atol=0)

@@ -487,8 +487,9 @@ __global__ __launch_bounds__(512) void monomial_tile_adjoint_kernel(
     if (o != before) g = gout[b * t.O + o];
     const Real v = uniform_value(hv[k]);
     const int64_t m = t.terms ? uniform64(h.terms[k]) : k;
-    const Real w = g * conjv(v);
-    Real mono = Real(1);
+    // a grouped table's monomial starts from its value (as forward: the product may fit where it alone does not)
+    const Real w = t.terms ? g * conjv(v) : g;
+    Real mono = t.terms ? Real(1) : v;
     int64_t zdeg = 0;  // exponents of the zero factors (dense: those past one factor make it two or more)
     int zc = 0;
     for_factors<DENSE>(t, h, m, [&](int c, int64_t e) {
