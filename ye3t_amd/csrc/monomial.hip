@@ -10,6 +10,7 @@
 // row); rows too wide for a tile, and the second order, on one thread per
 // (row, output) or per row.  No atomics, fixed order.  The tables are validated
 // by the caller (ye3t_amd.runtime checks them on the host).
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -426,7 +427,8 @@ __global__ __launch_bounds__(512) void monomial_tile_kernel(const Real* __restri
   const Real* const hv = static_cast<const Real*>(h.values);
   load_rows(x, b0, batch, t.D, xs);
   __syncthreads();
-  for (int64_t o = wave; o < t.O; o += waves) {
+  // a launch of few tiles shares the outputs among several workgroups a tile (blockIdx.y)
+  for (int64_t o = wave + int64_t(waves) * blockIdx.y; o < t.O; o += int64_t(waves) * gridDim.y) {
     const int64_t k1 = uniform64(h.offsets[o + 1]);
     Real acc = Real(0);
     for (int64_t k = uniform64(h.offsets[o]); k < k1; ++k) {
@@ -443,8 +445,9 @@ __global__ __launch_bounds__(512) void monomial_tile_kernel(const Real* __restri
 
 // Input gradient, with the zero-factor rules of monomial_gradient (dense: a
 // single zero factor of exponent one takes the cofactor) and of
-// sparse_monomial_adjoint_kernel, which are one: a zero degree of one.
-template <bool DENSE, bool HELD, typename Real>
+// sparse_monomial_adjoint_kernel, which are one: a zero degree of one.  SHARED:
+// coefficients name their monomials.
+template <bool DENSE, bool HELD, bool SHARED, typename Real>
 __global__ __launch_bounds__(512) void monomial_tile_adjoint_kernel(
     const Real* __restrict__ gout, const Real* __restrict__ x, int64_t batch, MonomialTable t,
     const int64_t* __restrict__ offsets, const Real* __restrict__ values, Real* __restrict__ gin) {
@@ -486,10 +489,10 @@ __global__ __launch_bounds__(512) void monomial_tile_adjoint_kernel(
     }
     if (o != before) g = gout[b * t.O + o];
     const Real v = uniform_value(hv[k]);
-    const int64_t m = t.terms ? uniform64(h.terms[k]) : k;
+    const int64_t m = SHARED ? uniform64(h.terms[k]) : k;
     // a grouped table's monomial starts from its value (as forward: the product may fit where it alone does not)
-    const Real w = t.terms ? g * conjv(v) : g;
-    Real mono = t.terms ? Real(1) : v;
+    const Real w = SHARED ? g * conjv(v) : g;
+    Real mono = SHARED ? Real(1) : v;
     int64_t zdeg = 0;  // exponents of the zero factors (dense: those past one factor make it two or more)
     int zc = 0;
     for_factors<DENSE>(t, h, m, [&](int c, int64_t e) {
@@ -531,34 +534,37 @@ int launch_tiles(const Real* gout, const Real* x, int64_t batch, const MonomialT
   while (waves > 0 && rows * size_t(1 + (gout ? waves : 0)) > kTileLds) waves /= 2;
   if (waves == 0) return YE3T_EUNSUPPORTED;
   if (!gout && t.O < waves) waves = int(t.O);
+  // one gradient copy only: a wave a tile, no faster than a thread a row unless the tile is full (one row of 100
+  // fp32 components, 1000 coefficients: 1136 us by the thread, 1458 here)
+  if (gout && waves == 1 && batch < kTileRows) return YE3T_EUNSUPPORTED;
   const size_t held = held_bytes(t, sizeof(Real));
   const bool hold = held <= kTableLds;
   const size_t lds = rows * size_t(1 + (gout ? waves : 0)) + (hold ? held : 0);
-  const dim3 grid{unsigned(tiles)}, block{unsigned(64 * waves)};
-  auto launch = [&](auto dense, auto keep) {
-    if (gout) {
-      auto* const kernel = &monomial_tile_adjoint_kernel<dense.value, keep.value, Real>;
+  // forward: up to two workgroups a compute unit, each with its share of a tile's outputs
+  int64_t split = gout ? 1 : std::min<int64_t>((t.O + waves - 1) / waves, 512 / tiles);
+  if (split < 1) split = 1;
+  const dim3 grid{unsigned(tiles), unsigned(split)}, block{unsigned(64 * waves)};
+  auto launch = [&](auto dense, auto keep, auto shared) {
+    auto start = [&](auto* kernel, const char* name, auto... args) {
       if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess) {
         (void)hipGetLastError();
         return int(YE3T_EUNSUPPORTED);
       }
-      hipLaunchKernelGGL((monomial_tile_adjoint_kernel<dense.value, keep.value, Real>), grid, block, lds, s, gout, x,
-                         batch, t, offsets, values, out);
-      return check_launch("monomial_tile_adjoint_kernel");
-    }
-    auto* const kernel = &monomial_tile_kernel<dense.value, keep.value, Real>;
-    if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess) {
-      (void)hipGetLastError();
-      return int(YE3T_EUNSUPPORTED);
-    }
-    hipLaunchKernelGGL((monomial_tile_kernel<dense.value, keep.value, Real>), grid, block, lds, s, x, batch, t, offsets,
-                       values, out);
-    return check_launch("monomial_tile_kernel");
+      hipLaunchKernelGGL(kernel, grid, block, lds, s, args...);
+      return check_launch(name);
+    };
+    if (gout)
+      return start(&monomial_tile_adjoint_kernel<dense.value, keep.value, shared.value, Real>,
+                   "monomial_tile_adjoint_kernel", gout, x, batch, t, offsets, values, out);
+    return start(&monomial_tile_kernel<dense.value, keep.value, Real>, "monomial_tile_kernel", x, batch, t, offsets,
+                 values, out);
   };
-  if (t.counts) return hold ? launch(std::true_type{}, std::true_type{}) : launch(std::true_type{}, std::false_type{});
-  return hold ? launch(std::false_type{}, std::true_type{}) : launch(std::false_type{}, std::false_type{});
+  const std::true_type yes;
+  const std::false_type no;
+  if (!t.counts) return hold ? launch(no, yes, yes) : launch(no, no, yes);
+  if (t.terms) return hold ? launch(yes, yes, yes) : launch(yes, no, yes);
+  return hold ? launch(yes, yes, no) : launch(yes, no, no);
 }
 
 int launch_tiles(int dtype, const void* gout, const void* x, int64_t batch, const MonomialTable& t,
