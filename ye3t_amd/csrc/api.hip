@@ -109,24 +109,26 @@ __global__ __launch_bounds__(kRadialRows) void radial_table_kernel(const Real* _
   constexpr int P = NR | 1;  // odd: consecutive rows start in different banks
   __shared__ Real vt[kRadialRows * P];
   __shared__ Real dt[DERIVS ? kRadialRows * P : 1];
-  const int64_t e0 = int64_t(blockIdx.x) * kRadialRows;
-  const int rows = E - e0 < kRadialRows ? int(E - e0) : kRadialRows;
   const int t = threadIdx.x;
-  if (t < rows) {
-    // The basis is evaluated in fp64 for both storage types: the Chebyshev
-    // recurrence amplifies rounding of the warped variable by ~n^2.
-    double v[NR], d[NR];
-    cheb_exp_cos_row<double, DERIVS>(double(radii[e0 + t]), double(cutoffs[e0 + t]), double(lambdas[e0 + t]), NR - 1,
-                                     v, d);
+  for (int64_t e0 = int64_t(blockIdx.x) * kRadialRows; e0 < E; e0 += int64_t(gridDim.x) * kRadialRows) {
+    const int rows = E - e0 < kRadialRows ? int(E - e0) : kRadialRows;
+    if (t < rows) {
+      // The basis is evaluated in fp64 for both storage types: the Chebyshev
+      // recurrence amplifies rounding of the warped variable by ~n^2.
+      double v[NR], d[NR];
+      cheb_exp_cos_row<double, DERIVS>(double(radii[e0 + t]), double(cutoffs[e0 + t]), double(lambdas[e0 + t]), NR - 1,
+                                       v, d);
 #pragma unroll
-    for (int n = 0; n < NR; ++n) {
-      vt[t * P + n] = Real(v[n]);
-      if (DERIVS) dt[t * P + n] = Real(d[n]);
+      for (int n = 0; n < NR; ++n) {
+        vt[t * P + n] = Real(v[n]);
+        if (DERIVS) dt[t * P + n] = Real(d[n]);
+      }
     }
+    __syncthreads();
+    copy_rows<NR, P>(vt, rows, values + e0 * NR);
+    if (DERIVS) copy_rows<NR, P>(dt, rows, derivs + e0 * NR);
+    __syncthreads();  // the tile is read before the next one is written
   }
-  __syncthreads();
-  copy_rows<NR, P>(vt, rows, values + e0 * NR);
-  if (DERIVS) copy_rows<NR, P>(dt, rows, derivs + e0 * NR);
 }
 
 template <int NR, typename Real>
@@ -135,7 +137,7 @@ int launch_radial(int nr, const Real* radii, const Real* cutoffs, const Real* la
   if constexpr (NR < 16) {
     if (nr > NR) return launch_radial<NR + 1>(nr, radii, cutoffs, lambdas, E, values, derivs, s);
   }
-  const dim3 grid{unsigned((E + kRadialRows - 1) / kRadialRows)};
+  const dim3 grid{grid_for(E, kRadialRows)};
   if (derivs) {
     hipLaunchKernelGGL((radial_table_kernel<NR, true, Real>), grid, dim3(kRadialRows), 0, s, radii, cutoffs, lambdas, E,
                        values, derivs);
@@ -283,7 +285,7 @@ int launch_channels(const Real* rv, const Real* rd, const Real* av, const Real* 
   if (held && tile > fit) tile = fit;
   tile = tile < 2 ? 2 : tile / 2 * 2;
   const int64_t groups = (E + tile - 1) / tile;
-  YE3T_REQUIRE(groups <= INT32_MAX, "too many edges for one launch");
+  YE3T_REQUIRE(fits_grid(groups, kChannelThreads), "too many edges for one launch");  // from 500 GB of rows on
   if (held) {
     hipLaunchKernelGGL((scheduled_channels_kernel<true, Real>), dim3(unsigned(groups)), dim3(kChannelThreads),
                        size_t(K) * sizeof(ChannelSchedule<Real>) + size_t(tile * row), s, rv, rd, av, ad, dir, types,
@@ -417,12 +419,15 @@ __global__ __launch_bounds__(256) void sph_tile_kernel(const Real* __restrict__ 
   if (GRAD) copy_rows<3 * W, GP>(gt, rows, grads + e0 * 3 * W);
 }
 
+// edges of a tile
+constexpr int sph_tile_edges(int lmax, size_t elem) { return lmax > 6 && elem == 8 ? 32 : 64; }
+
 template <int LMAX, typename Real>
 int launch_sph_tile(int lmax, const Real* vec, int64_t E, double eps, Real* values, Real* grads, hipStream_t s) {
   if constexpr (LMAX < 8) {
     if (lmax > LMAX) return launch_sph_tile<LMAX + 1>(lmax, vec, E, eps, values, grads, s);
   }
-  constexpr int T = LMAX > 6 && sizeof(Real) == 8 ? 32 : 64;
+  constexpr int T = sph_tile_edges(LMAX, sizeof(Real));
   const dim3 grid{unsigned((E + T - 1) / T)};
   if (grads) {
     hipLaunchKernelGGL((sph_tile_kernel<LMAX, true, T, Real>), grid, dim3(256), 0, s, vec, E, eps, norm_table(), values,
@@ -434,8 +439,8 @@ int launch_sph_tile(int lmax, const Real* vec, int64_t E, double eps, Real* valu
   return check_launch("sph_tile_kernel");
 }
 
-// The same table for any l_max (l_max 9 and above): one lane per edge, the
-// recurrences in scratch.
+// The same table for any l_max and edge count (l_max 9 and above, and more edges
+// than one grid has tiles): one lane per edge, the recurrences in scratch.
 template <typename Real>
 __global__ __launch_bounds__(128) void real_sph_table_kernel(const Real* __restrict__ vec, int64_t E, int lmax,
                                                              double eps, NormTable nt, Real* __restrict__ values,
@@ -699,7 +704,6 @@ int ye3t_hip_radial_table(int dtype, const void* radii, const void* cutoffs, con
   YE3T_REQUIRE(n_max >= 0 && n_max < 16, "max_radial_index must be in [0, 15], got %lld", (long long)n_max);
   if (E == 0) return YE3T_OK;
   YE3T_REQUIRE(radii && cutoffs && lambdas && values, "NULL input or output");
-  YE3T_REQUIRE((E + kRadialRows - 1) / kRadialRows <= INT32_MAX, "too many edges for one launch");
   if (dtype == YE3T_F64)
     return launch_radial<1>(int(n_max) + 1, (const double*)radii, (const double*)cutoffs, (const double*)lambdas, E,
                             (double*)values, (double*)derivs, as_stream(stream));
@@ -751,7 +755,8 @@ int ye3t_hip_real_sph_table(int dtype, const void* vec, int64_t E, int64_t lmax,
   YE3T_REQUIRE(lmax >= 0 && lmax <= kMaxL, "maximum_angular_momentum must be in [0, %d]", kMaxL);
   if (E == 0) return YE3T_OK;
   YE3T_REQUIRE(vec && values, "NULL input or output");
-  if (lmax <= 8 && E <= int64_t(INT32_MAX) * 32) {
+  const int tile = sph_tile_edges(int(lmax), dtype == YE3T_F64 ? 8 : 4);
+  if (lmax <= 8 && fits_grid((E + tile - 1) / tile, 256)) {
     if (dtype == YE3T_F64)
       return launch_sph_tile<0>(int(lmax), (const double*)vec, E, eps, (double*)values, (double*)grads, as_stream(stream));
     if (dtype == YE3T_F32)

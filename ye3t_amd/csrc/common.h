@@ -36,6 +36,10 @@ inline int check_launch(const char* what) {
   return YE3T_OK;
 }
 
+// Whether one grid axis holds `groups` workgroups of `threads`: HIP counts its
+// work items in 32 bits.
+inline bool fits_grid(int64_t groups, int threads) { return groups <= int64_t(0xFFFFFFFF) / threads; }
+
 inline hipStream_t as_stream(ye3t_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
 // ---- device math, overloaded for float / double ----------------------------

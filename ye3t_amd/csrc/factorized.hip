@@ -946,11 +946,11 @@ int fa_launch(const ye3t_hip_factorized_angular_plan* p, int op, const void* pac
   const int64_t per = p->max_workspace * int64_t(sizeof(T)) * copies;
   int units = 64;
   while (units > 1 && per * units > kSortedLds) units /= 2;
-  if (p->sorted && op != 2 && per * units <= 64 * 1024 && units >= p->max_sources && batch <= (int64_t(1) << 40)) {
-    const int64_t lanes = op == 0 ? units / p->max_sources : units;  // samples, or (sample, source) pairs, of a wave
-    const int64_t work = op == 0 ? batch : batch * p->max_sources;
-    const int64_t groups = (work + lanes - 1) / lanes;
-    YE3T_REQUIRE(groups <= int64_t(0x7FFFFFFF), "batch too large for one launch");
+  const int64_t lanes = op == 0 ? units / p->max_sources : units;  // samples, or (sample, source) pairs, of a wave
+  const int64_t work = op == 0 ? batch : batch * p->max_sources;
+  const int64_t groups = lanes > 0 ? (work + lanes - 1) / lanes : 0;
+  if (p->sorted && op != 2 && per * units <= 64 * 1024 && units >= p->max_sources && batch <= (int64_t(1) << 40) &&
+      fits_grid(groups, 64)) {
     const dim3 blocks(unsigned(groups), unsigned(p->segment_count));
     const T* value = static_cast<const T*>(p->sorted_values);
     const T* proj = static_cast<const T*>(p->projection);

@@ -523,17 +523,19 @@ __global__ __launch_bounds__(512) void monomial_tile_adjoint_kernel(
 }
 
 // Launches a tile kernel; YE3T_EUNSUPPORTED, with nothing launched, where a
-// tile of rows (and one wave's gradients) does not fit in kTileLds.
+// tile of rows (and one wave's gradients) does not fit in kTileLds, or the tiles
+// not in one grid.
 template <typename Real>
 int launch_tiles(const Real* gout, const Real* x, int64_t batch, const MonomialTable& t, const int64_t* offsets,
                  const Real* values, Real* out, hipStream_t s) {
   const size_t rows = size_t(t.D) * kTileRows * sizeof(Real);
   const int64_t tiles = (batch + kTileRows - 1) / kTileRows;
-  if (t.D < 1 || t.O < 1 || t.D > 1024 || tiles > INT32_MAX) return YE3T_EUNSUPPORTED;
+  if (t.D < 1 || t.O < 1 || t.D > 1024) return YE3T_EUNSUPPORTED;
   int waves = 8;
   while (waves > 0 && rows * size_t(1 + (gout ? waves : 0)) > kTileLds) waves /= 2;
   if (waves == 0) return YE3T_EUNSUPPORTED;
   if (!gout && t.O < waves) waves = int(t.O);
+  if (!fits_grid(tiles, 64 * waves)) return YE3T_EUNSUPPORTED;  // the kernels of one thread a row take any batch
   // one gradient copy only: a wave a tile, no faster than a thread a row unless the tile is full (one row of 100
   // fp32 components, 1000 coefficients: 1136 us by the thread, 1458 here)
   if (gout && waves == 1 && batch < kTileRows) return YE3T_EUNSUPPORTED;
