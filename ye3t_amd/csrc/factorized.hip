@@ -359,20 +359,43 @@ __global__ __launch_bounds__(64) void fa_sorted_forward_kernel(const FATables* _
   T* const ws = reinterpret_cast<T*>(fa_smem) + lane;
   if (on) fa_sorted_replay(t, value, packed + b * t.in_stride + t.in_off + s * t.input_dim, ws, units);
   __syncthreads();  // one wave: a sample's sources are its neighbouring lanes
-  if (!on || s != 0) return;
+  if (!on) return;
   const T* proj = proj_all + t.proj_off;
   T* orow = out + b * t.out_stride + t.out_off;
+  // the values of a root go over the sample's lanes; of one or two, one does
+  // them all, for which the projection is wave-uniform.  20 000 samples, three
+  // l = 2 slots to L = 2, fp64, eight projections: two sources 56 us by both
+  // lanes, 45 by one; sixteen 155 by all, 553 by one (a lane a sample before the
+  // tables were sorted: 933)
+  const T* const first = ws - s;
   for (int r = 0; r < t.root_count; ++r) {
     const int rn = at(t.roots, r);
     const int roff = at(t.node_offsets, rn), rd = at(t.node_dims, rn);
     const int ps = at(t.root_ps, r), pd = at(t.root_pd, r);
     T* blk = orow + at(t.root_oo, r);
-    for (int p = 0; p < pd; ++p, blk += rd) {
-      for (int m = 0; m < rd; ++m) {
-        T acc = O::zero();
-        for (int k = 0; k < S; ++k)
-          acc = O::add(acc, O::mul(ws[(roff + m) * units + k], proj[k * t.proj_dim + ps + p]));
-        blk[m] = acc;
+    if (S <= 2) {
+      for (int p = 0; s == 0 && p < pd; ++p, blk += rd) {
+        for (int m = 0; m < rd; ++m) {
+          T acc = O::zero();
+          for (int k = 0; k < S; ++k)
+            acc = O::add(acc, O::mul(ws[(roff + m) * units + k], proj[k * t.proj_dim + ps + p]));
+          blk[m] = acc;
+        }
+      }
+      continue;
+    }
+    const int dp = S / rd, dm = S - dp * rd;
+    for (int p = s / rd, m = s - p * rd; p < pd;) {
+      const T* const v = first + (roff + m) * units;
+      const T* const w = proj + ps + p;
+      T acc = O::zero();
+      for (int k = 0; k < S; ++k) acc = O::add(acc, O::mul(v[k], w[k * t.proj_dim]));
+      blk[p * rd + m] = acc;
+      p += dp;
+      m += dm;
+      if (m >= rd) {
+        m -= rd;
+        ++p;
       }
     }
   }
