@@ -64,3 +64,18 @@ def test_radial_table_tiles(gpu, dtype, edges):
         assert column_rel_error(d.cpu().numpy(), d_ref) < TOL[dtype], n_max
         v0, none = native.radial_table(r, rc, lam, n_max, with_derivative=False)
         assert none is None and torch.equal(v0, v)
+
+
+@pytest.mark.parametrize("l_max", [0, 3, 6, 8])
+def test_harmonic_gradient_of_a_length_that_overflows(gpu, l_max):
+    """A vector whose squares overflow: direction zero and gradient zero, as the general kernel (l_max 9) has it."""
+    flush(f"harmonic table, |v| beyond the square root of the largest number, l_max {l_max}")
+    import torch
+
+    v = torch.tensor([[1e160, -2e160, 3e155], [0.3, -0.4, 0.5], [0.0, 2e170, 0.0]], dtype=torch.float64, device=gpu)
+    width = (l_max + 1) ** 2
+    y, g = native.real_sph_table(v, l_max)
+    y9, g9 = native.real_sph_table(v, 9)
+    assert bool((g[[0, 2]] == 0).all()) and bool((g9[[0, 2]] == 0).all())
+    assert torch.allclose(y, y9[:, :width], rtol=1e-12, atol=1e-14)
+    assert torch.allclose(g[1], g9[1, :width], rtol=1e-12, atol=1e-12)

@@ -320,6 +320,7 @@ __device__ inline void sph_tile_rows(const double (&u)[3], double sr, bool proje
   double cr = 1.0, ci = 0.0, pr = 1.0, pi = 0.0;  // (x + i y)^m and ^(m-1)
   double qmm = 1.0;                               // Q_m^m
   const double inv = 1.0 / sr;
+  const double rem = sr == HUGE_VAL ? 0.0 : sr;  // a length that overflows has gradient zero
   // the gradient (gx, gy, gz) w.r.t. u of component k, taken to the vector and stored
   auto put = [&](int k, double gx, double gy, double gz) {
     if (project) {
@@ -331,7 +332,7 @@ __device__ inline void sph_tile_rows(const double (&u)[3], double sr, bool proje
     // g / sr, the reciprocal's product corrected by its remainder
     auto over = [&](double g) {
       const double q = g * inv;
-      return fma(fma(-q, sr, g), inv, q);
+      return fma(fma(-q, rem, g), inv, q);
     };
     grow[3 * k] = Real(over(gx));
     grow[3 * k + 1] = Real(over(gy));
