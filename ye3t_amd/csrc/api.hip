@@ -158,16 +158,20 @@ int launch_radial(int nr, const Real* radii, const Real* cutoffs, const Real* la
 // the kernel clamps them into the tables rather than faulting.
 //
 // Four values are written for each of E K outputs; those writes bound it.  A
-// workgroup takes whole edges, about 4 096 outputs, with their table rows and the
-// schedule in LDS (an output reads ten values, each of them shared by a row of
-// others) and lane = output; the three components of a wave's 64 outputs go
-// through LDS too, so that every store is contiguous.  240 000 edges x 144
+// workgroup takes whole edges, up to about 4 096 outputs, with their table rows
+// and the schedule in LDS (an output reads ten values, each of them shared by a
+// row of others) and lane = output; the three components of a wave's 64 outputs
+// go through LDS too, so that every store is contiguous.  240 000 edges x 144
 // channels in fp64 (1.1 GB written): 425 -> 250 us (one thread an output with
 // a 64-bit division and 24-byte strided stores before; 354 us with the rows
-// read from memory).
+// read from memory).  Fewer outputs a workgroup where that leaves compute units
+// without one: 1 000 edges x 144 11.5 -> 5.3 us (one thread an output: 5.3).
+// Rows are held only where the channels read most of them: 100 channels of
+// 1 000 harmonics, fp32, 100 000 edges, 907 us held, 223 from memory; 12
+// channels of 3 and 4, 200 000 edges, 22 and 24.
 constexpr int kChannelThreads = 256;
 constexpr int64_t kChannelTable = 1024;     // channels whose schedule is held in LDS (24 KB)
-constexpr int64_t kChannelRows = 32 * 1024;  // bytes of edge rows held in LDS
+constexpr int64_t kChannelRows = 16 * 1024;  // bytes of edge rows held in LDS: six workgroups a compute unit
 
 template <typename Real>
 struct ChannelSchedule {
@@ -182,7 +186,7 @@ __global__ __launch_bounds__(kChannelThreads) void scheduled_channels_kernel(
     const Real* __restrict__ rv, const Real* __restrict__ rd, const Real* __restrict__ av,
     const Real* __restrict__ ad, const Real* __restrict__ dir, const int64_t* __restrict__ edge_types,
     const int64_t* __restrict__ cri, const int64_t* __restrict__ cai, const int64_t* __restrict__ ctype,
-    const Real* __restrict__ cscale, int64_t E, int64_t NR, int64_t NA, int64_t K, int64_t tile,
+    const Real* __restrict__ cscale, int64_t E, int64_t NR, int64_t NA, int64_t K, int64_t tile, int64_t part,
     Real* __restrict__ values, Real* __restrict__ derivs) {
 #pragma clang fp contract(off)
   constexpr int V = 16 / int(sizeof(Real));
@@ -220,15 +224,16 @@ __global__ __launch_bounds__(kChannelThreads) void scheduled_channels_kernel(
     hold(sdir, dir + e0 * 3, edges * 3);
     __syncthreads();
   }
-  const int64_t outputs = edges * K;
+  const int64_t first = int64_t(blockIdx.y) * part;  // this workgroup's part of the tile's outputs
+  const int64_t outputs = edges * K < first + part ? edges * K : first + part;
   const int64_t o0 = e0 * K;
   const int lane = threadIdx.x & 63;
   Real* const mine = stage[threadIdx.x >> 6];
   const bool aligned = reinterpret_cast<uintptr_t>(derivs + 3 * o0) % 16 == 0;
   // the lane's channel and edge (of the tile) advance by 256 outputs a step
   const int dk = int(kChannelThreads % K), de = int(kChannelThreads / K);
-  int64_t e = int64_t(threadIdx.x) / K, k = int64_t(threadIdx.x) % K;
-  for (int64_t w = threadIdx.x - lane; w < outputs; w += kChannelThreads) {
+  int64_t e = (first + threadIdx.x) / K, k = first + threadIdx.x - e * K;
+  for (int64_t w = first + threadIdx.x - lane; w < outputs; w += kChannelThreads) {
     const int left = outputs - w < 64 ? int(outputs - w) : 64;  // outputs of this wave's step
     if (lane < left) {
       const ChannelSchedule<Real> c = HELD ? table[k] : schedule(k);
@@ -276,23 +281,35 @@ int launch_channels(const Real* rv, const Real* rd, const Real* av, const Real* 
                     const int64_t* types, const int64_t* cri, const int64_t* cai, const int64_t* ctype,
                     const Real* cscale, int64_t E, int64_t NR, int64_t NA, int64_t K, Real* values, Real* derivs,
                     hipStream_t s) {
-  // edges of a workgroup: about 4 096 outputs, as far as their rows fit, and an
-  // even number (rows of three fp64 values start on 16 bytes every second output)
-  const int64_t row = (2 * NR + 4 * NA + 3) * int64_t(sizeof(Real)) + 8;
-  const int64_t fit = kChannelRows / row;
-  const bool held = K <= kChannelTable && fit >= 2;
-  int64_t tile = 4096 / K;
-  if (held && tile > fit) tile = fit;
+  // outputs of a workgroup: 4 096, or fewer where that leaves compute units
+  // without one; edges: as many as have those, an even number (rows of three
+  // fp64 values start on 16 bytes every second output), as far as their rows
+  // fit; a tile of two edges with more outputs than that is shared by several
+  int64_t part = (E * K / 1024 + kChannelThreads - 1) / kChannelThreads * kChannelThreads;
+  part = part < kChannelThreads ? kChannelThreads : (part > 4096 ? 4096 : part);
+  int64_t tile = part / K;
   tile = tile < 2 ? 2 : tile / 2 * 2;
+  const int64_t parts = tile * K <= part + part / 2 ? 1 : (tile * K + part - 1) / part;
+  if (parts == 1) part = tile * K;
+  // held: whole edges, and rows of which the channels read most
+  const int64_t row = (2 * NR + 4 * NA + 3) * int64_t(sizeof(Real)) + 8;
+  const int64_t fit = kChannelRows / row / 2 * 2;
+  const bool held = parts == 1 && K <= kChannelTable && fit >= 2 && 2 * NR + 4 * NA <= 8 * K;
+  if (held && tile > fit) {
+    tile = fit;
+    part = tile * K;
+  }
   const int64_t groups = (E + tile - 1) / tile;
   YE3T_REQUIRE(fits_grid(groups, kChannelThreads), "too many edges for one launch");  // from 500 GB of rows on
+  YE3T_REQUIRE(parts <= 65535, "too many channels for one launch");
+  const dim3 grid{unsigned(groups), unsigned(parts)};
   if (held) {
-    hipLaunchKernelGGL((scheduled_channels_kernel<true, Real>), dim3(unsigned(groups)), dim3(kChannelThreads),
+    hipLaunchKernelGGL((scheduled_channels_kernel<true, Real>), grid, dim3(kChannelThreads),
                        size_t(K) * sizeof(ChannelSchedule<Real>) + size_t(tile * row), s, rv, rd, av, ad, dir, types,
-                       cri, cai, ctype, cscale, E, NR, NA, K, tile, values, derivs);
+                       cri, cai, ctype, cscale, E, NR, NA, K, tile, part, values, derivs);
   } else {
-    hipLaunchKernelGGL((scheduled_channels_kernel<false, Real>), dim3(unsigned(groups)), dim3(kChannelThreads), 0, s,
-                       rv, rd, av, ad, dir, types, cri, cai, ctype, cscale, E, NR, NA, K, tile, values, derivs);
+    hipLaunchKernelGGL((scheduled_channels_kernel<false, Real>), grid, dim3(kChannelThreads), 0, s, rv, rd, av, ad, dir,
+                       types, cri, cai, ctype, cscale, E, NR, NA, K, tile, part, values, derivs);
   }
   return check_launch("scheduled_channels_kernel");
 }
