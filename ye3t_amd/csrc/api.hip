@@ -590,27 +590,29 @@ __global__ __launch_bounds__(256) void csr_offsets_kernel(const int64_t* __restr
 }
 
 // Gather of centre-row adjoints to edge rows.  A workgroup copies 256 vectors
-// at a time (V = 16 bytes when the rows allow it), eight steps over consecutive
+// at a time (V = 16 bytes when the rows allow it), STEPS steps over consecutive
 // vectors of the edge rows with every step's read requested before the first
 // write; the output is streamed with non-temporal stores (written once, not
 // re-read here).  Centres are validated by the caller; an index outside [0, N)
-// is clamped so that no access leaves the array.  240 000 edges x 144 channels
-// in fp64 (276 MB written): 92 -> 67 us (one step a workgroup before).
-constexpr int kGatherSteps = 8;
+// is clamped so that no access leaves the array.  Several steps where the copies
+// do not fit the caches any more, one where more workgroups count: fp64, 144
+// channels, 240 000 edges (17 million vectors) 60 us by one step, 45 by four, 51
+// by eight; 20 000 edges (1.4 million) 5.5, 6.3 and 7.5; 225 channels (single
+// values), 100 000 edges (23 million) 53, 45 and 40.
+constexpr int64_t kGatherLarge = 5000000;  // vectors
 
-template <typename V>
+template <int STEPS, typename Index, typename V>
 __global__ __launch_bounds__(256) void density_adjoint_kernel(const V* __restrict__ adj,
                                                               const int64_t* __restrict__ centers, int64_t E,
                                                               int64_t CV, int64_t N, V* __restrict__ out) {
   const int64_t total = E * CV;
   const int64_t dc = 256 % CV, de = 256 / CV;
-  for (int64_t x0 = int64_t(blockIdx.x) * (256 * kGatherSteps); x0 < total;
-       x0 += int64_t(gridDim.x) * (256 * kGatherSteps)) {
+  for (int64_t x0 = int64_t(blockIdx.x) * (256 * STEPS); x0 < total; x0 += int64_t(gridDim.x) * (256 * STEPS)) {
     const int64_t x = x0 + threadIdx.x;
-    int64_t e = x / CV, c = x - e * CV;
-    V v[kGatherSteps];
+    int64_t e = Index(x) / Index(CV), c = x - e * CV;
+    V v[STEPS];
 #pragma unroll
-    for (int k = 0; k < kGatherSteps; ++k) {
+    for (int k = 0; k < STEPS; ++k) {
       if (x + 256 * k < total) {
         int64_t i = centers[e];
         i = i < 0 ? 0 : (i >= N ? N - 1 : i);
@@ -624,9 +626,22 @@ __global__ __launch_bounds__(256) void density_adjoint_kernel(const V* __restric
       }
     }
 #pragma unroll
-    for (int k = 0; k < kGatherSteps; ++k)
+    for (int k = 0; k < STEPS; ++k)
       if (x + 256 * k < total) __builtin_nontemporal_store(v[k], out + x + 256 * k);
   }
+}
+
+template <typename V>
+int launch_gather(const void* adj, const int64_t* centers, int64_t E, int64_t CV, int64_t N, void* out, hipStream_t s) {
+  constexpr int kSteps = sizeof(V) == 16 ? 4 : 8;
+  if (E * CV >= kGatherLarge) {
+    hipLaunchKernelGGL((density_adjoint_kernel<kSteps, int64_t, V>), dim3(grid_for(E * CV, 256 * kSteps)), dim3(256), 0,
+                       s, static_cast<const V*>(adj), centers, E, CV, N, static_cast<V*>(out));
+  } else {
+    hipLaunchKernelGGL((density_adjoint_kernel<1, uint32_t, V>), dim3(grid_for(E * CV, 256)), dim3(256), 0, s,
+                       static_cast<const V*>(adj), centers, E, CV, N, static_cast<V*>(out));
+  }
+  return check_launch("density_adjoint_kernel");
 }
 
 // Range checks of index inputs in one pass over them, one grid row an array:
@@ -872,18 +887,9 @@ int ye3t_hip_density_accumulate_adjoint(int dtype, const void* adj, const int64_
                    reinterpret_cast<uintptr_t>(out) % 16 == 0;
   const hipStream_t s = as_stream(stream);
   const int64_t CV = vec ? int64_t(size_t(C) * elem / 16) : C;
-  const unsigned grid = grid_for(E * CV, 256 * kGatherSteps);
-  if (vec) {
-    hipLaunchKernelGGL(density_adjoint_kernel<f32x4>, dim3(grid), dim3(256), 0, s, (const f32x4*)adj, centers, E,
-                       CV, N, (f32x4*)out);
-  } else if (dtype == YE3T_F64) {
-    hipLaunchKernelGGL(density_adjoint_kernel<double>, dim3(grid), dim3(256), 0, s, (const double*)adj, centers, E,
-                       CV, N, (double*)out);
-  } else {
-    hipLaunchKernelGGL(density_adjoint_kernel<float>, dim3(grid), dim3(256), 0, s, (const float*)adj, centers, E,
-                       CV, N, (float*)out);
-  }
-  return check_launch("density_adjoint_kernel");
+  if (vec) return launch_gather<f32x4>(adj, centers, E, CV, N, out, s);
+  if (dtype == YE3T_F64) return launch_gather<double>(adj, centers, E, CV, N, out, s);
+  return launch_gather<float>(adj, centers, E, CV, N, out, s);
 }
 
 }  // extern "C"
