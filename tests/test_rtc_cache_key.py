@@ -40,3 +40,23 @@ def test_compile_lands_under_the_key(tmp_path, monkeypatch):
     assert path.exists() and path.read_bytes() == blob
     assert blob[:4] == b"\x7fELF"
     assert len(os.listdir(tmp_path)) == 1
+
+
+def test_several_sources_compile_in_children(tmp_path, monkeypatch):
+    """Code objects left in the cache by other processes, in the order asked for; what is wrong with a source is
+    raised."""
+    import pytest
+
+    sources = [SRC.replace("void k(", f"void k{k}(") for k in (3, 4, 5, 3)]
+    monkeypatch.setenv("YE3T_AMD_JIT_CACHE", str(tmp_path))
+    found = []
+    whole = native.rtc_compile
+    monkeypatch.setattr(native, "rtc_compile", lambda src: found.append(
+        (tmp_path / (native.rtc_cache_key(src) + ".co")).exists()) or whole(src))
+    blobs = native.rtc_compile_many(sources)
+    assert found == [True] * 4  # this process only reads
+    assert blobs[0] == blobs[3] and len({bytes(b) for b in blobs}) == 3
+    for blob, k in zip(blobs, (3, 4, 5, 3)):
+        assert native.code_object_kernel_info(blob, f"k{k}")["private_segment_bytes"] == 0
+    with pytest.raises(RuntimeError, match="no_such_type"):
+        native.rtc_compile_many([SRC.replace("2.0", "7.0"), SRC.replace("double", "no_such_type")])

@@ -60,11 +60,10 @@ def fit_parts_to_scratch(make, live, kernel, compile_all=None):
     each code object) needs at most ``native.part_private_limit()`` bytes of
     scratch per lane; the attach entry points refuse any part above it.
     ``make(n)`` returns ``[(source, meta), ...]``; ``compile_all(sources)``
-    returns their code objects (default: hipRTC through the JIT cache, one at
-    a time)."""
+    returns their code objects (default: ``native.rtc_compile_many``)."""
     limit = native.part_private_limit()
     if compile_all is None:
-        compile_all = lambda sources: [native.rtc_compile(src) for src in sources]  # noqa: E731
+        compile_all = native.rtc_compile_many
     while True:
         parts = make(live)
         codes = compile_all([src for src, _meta in parts])

@@ -5,7 +5,8 @@ generated kernel in parts (``codegen.generate_parts``, with the reverse sweep
 ``generate_adjoint_parts`` and the fused readout ``generate_readout_parts``),
 one hipRTC module per 9 chunks (64 for plans above 100 000 terms).  hipRTC
 compiles one module at a time per process (one to five minutes for a 64-chunk
-config-3 part), so the parts are spread over worker processes.  hipRTC needs
+config-3 part), so the parts are spread over child processes
+(``native.rtc_compile_many``, which a pipeline uses too).  hipRTC needs
 no GPU, so this runs on a build host; the code objects land in the JIT cache
 (``ye3t_amd/jit_cache`` unless ``YE3T_AMD_JIT_CACHE`` says otherwise), keyed by
 architecture, compiler fingerprint (hipRTC version, options, ABI) and source
@@ -16,11 +17,9 @@ architecture, compiler fingerprint (hipRTC version, options, ABI) and source
 """
 
 import argparse
-import multiprocessing
 import os
 import sys
 import time
-from concurrent.futures import ProcessPoolExecutor
 
 
 def precisions(cfg, dtype):
@@ -28,12 +27,6 @@ def precisions(cfg, dtype):
     accumulate = (cfg.accumulate if dtype == "f32" else None) or dtype
     density = (cfg.density_dtype if dtype == "f32" and accumulate == cfg.accumulate else None) or accumulate
     return accumulate, density
-
-
-def _compile(source):
-    from ye3t_amd.runtime import native
-
-    return native.rtc_compile(source)
 
 
 def prebuild(config_ids=(2, 3, 5), dtypes=None, workers=None, log=print):
@@ -62,19 +55,16 @@ def prebuild(config_ids=(2, 3, 5), dtypes=None, workers=None, log=print):
                                                     chunks_per_part=ADJOINT_PART_CHUNKS, grad_dtype=dtype,
                                                     in_dtype=density)
             t0 = time.time()
-            # worker processes (spawned: nothing of this process is inherited) compile in parallel;
             # parts above the library's scratch bound are regenerated in smaller chunks, as the
             # pipeline does (fit_parts_to_scratch)
-            with ProcessPoolExecutor(workers, mp_context=multiprocessing.get_context("spawn")) as pool:
-                compile_all = lambda sources: list(pool.map(_compile, sources))  # noqa: E731
-                parts = fit_parts_to_scratch(
-                    lambda n: generate_parts(plan, accumulate, max_live=n, chunks_per_part=per, out_dtype=dtype,
-                                             in_dtype=density), live, "ye3t_product_part", compile_all)
-                readout = fit_parts_to_scratch(
-                    lambda n: generate_readout_parts(plan, accumulate, max_live=n, chunks_per_part=per,
-                                                     in_dtype=density)[0], live, "ye3t_product_readout_part",
-                    compile_all)
-                compile_all([part[0] for part in adjoint])
+            compile_all = lambda sources: native.rtc_compile_many(sources, workers)  # noqa: E731
+            parts = fit_parts_to_scratch(
+                lambda n: generate_parts(plan, accumulate, max_live=n, chunks_per_part=per, out_dtype=dtype,
+                                         in_dtype=density), live, "ye3t_product_part", compile_all)
+            readout = fit_parts_to_scratch(
+                lambda n: generate_readout_parts(plan, accumulate, max_live=n, chunks_per_part=per,
+                                                 in_dtype=density)[0], live, "ye3t_product_readout_part", compile_all)
+            compile_all([part[0] for part in adjoint])
             log(f"config {cid} {dtype} (arithmetic {accumulate}, density {density}): {len(parts)} forward, "
                 f"{len(adjoint)} adjoint and {len(readout)} readout parts in {time.time() - t0:.1f} s "
                 f"-> {native._jit_cache_dir()}")

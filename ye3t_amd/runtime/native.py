@@ -1026,6 +1026,37 @@ def rtc_compile(source, name="ye3t_generated.hip", arch="gfx950"):
     return blob
 
 
+def rtc_compile_many(sources, workers=None):
+    """``rtc_compile`` of several sources.  hipRTC compiles one module at a time
+    in a process, so those that are not cached go to child processes, which leave
+    them in the cache (a part of a plan takes 10 to 60 seconds; config 3's 42 in
+    fp64 take 192 s with six workers).  A child that does not end well is made up
+    for here, which raises what is wrong with its source."""
+    import subprocess
+    import sys
+    from concurrent.futures import ThreadPoolExecutor
+
+    directory = _jit_cache_dir()
+    missing = [src for src in dict.fromkeys(sources)
+               if not os.path.exists(os.path.join(directory, rtc_cache_key(src) + ".co"))]
+    if len(missing) > 1 and sys.executable:
+        root = os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+        path = os.pathsep.join([root] + [p for p in (os.environ.get("PYTHONPATH"),) if p])
+        env = dict(os.environ, PYTHONPATH=path, YE3T_AMD_JIT_CACHE=directory)
+        code = "import sys; from ye3t_amd.runtime import native; native.rtc_compile(sys.stdin.read())"
+
+        def child(src):
+            try:
+                subprocess.run([sys.executable, "-c", code], input=src.encode(), env=env, stdout=subprocess.DEVNULL,
+                               stderr=subprocess.DEVNULL)
+            except OSError:
+                pass  # no process to be had
+
+        with ThreadPoolExecutor(max(1, min(workers or 12, os.cpu_count() or 1, len(missing)))) as pool:
+            list(pool.map(child, missing))
+    return [rtc_compile(src) for src in sources]
+
+
 def code_object_kernel_info(code, kernel_name):
     """``{"private_segment_bytes", "group_segment_bytes", "uses_dynamic_stack"}``
     of a kernel in a gfx950 code object, read on the host from its kernel
@@ -1143,10 +1174,8 @@ class ProductPlanHandle:
         self.generated = meta
 
     def attach_generated_parts(self, parts, workers=None):
-        """Compile (hipRTC, in parallel threads, cached on disk) and attach a
+        """Compile (hipRTC, in parallel processes, cached on disk) and attach a
         plan-specialised kernel in parts (``ye3t_amd.ace.codegen.generate_parts``)."""
-        from concurrent.futures import ThreadPoolExecutor
-
         first = 0
         for _source, meta in parts:
             if meta["feature_count"] != self.feature_count or meta["a_width"] != self.program["a_width"]:
@@ -1159,9 +1188,7 @@ class ProductPlanHandle:
             first = meta["last_output"]
         if first != self.feature_count:
             raise ValueError("generated parts do not cover every output")
-        workers = workers or min(16, os.cpu_count() or 1)
-        with ThreadPoolExecutor(max(1, workers)) as pool:
-            blobs = list(pool.map(lambda part: rtc_compile(part[0]), parts))
+        blobs = rtc_compile_many([part[0] for part in parts], workers)
         n = len(parts)
         self._part_code = [ctypes.create_string_buffer(b, len(b)) for b in blobs]
         codes = (_vp * n)(*[ctypes.cast(c, _vp) for c in self._part_code])
@@ -1175,16 +1202,12 @@ class ProductPlanHandle:
     def attach_adjoint_parts(self, parts, reduction, workers=None):
         """Compile and attach the reverse mode in parts
         (``ye3t_amd.ace.codegen.generate_adjoint_parts``)."""
-        from concurrent.futures import ThreadPoolExecutor
-
         for _source, meta in parts:
             if meta["feature_count"] != self.feature_count or meta["a_width"] != self.program["a_width"]:
                 raise ValueError("adjoint part does not match this plan")
             if meta["dtype"] != self.dtype or meta["grad_dtype"] != self.out_dtype or meta["in_dtype"] != self.in_dtype:
                 raise ValueError("adjoint part dtypes do not match this plan")
-        workers = workers or min(16, os.cpu_count() or 1)
-        with ThreadPoolExecutor(max(1, workers)) as pool:
-            blobs = list(pool.map(lambda part: rtc_compile(part[0]), parts))
+        blobs = rtc_compile_many([part[0] for part in parts], workers)
         n = len(parts)
         self._adjoint_part_code = [ctypes.create_string_buffer(b, len(b)) for b in blobs]
         codes = (_vp * n)(*[ctypes.cast(c, _vp) for c in self._adjoint_part_code])
@@ -1202,16 +1225,12 @@ class ProductPlanHandle:
     def attach_readout_parts(self, parts, workers=None):
         """Compile and attach the fused linear readout in parts
         (``ye3t_amd.ace.codegen.generate_readout_parts``)."""
-        from concurrent.futures import ThreadPoolExecutor
-
         for _source, meta in parts:
             if meta["feature_count"] != self.feature_count or meta["a_width"] != self.program["a_width"]:
                 raise ValueError("readout part does not match this plan")
             if meta["dtype"] != self.dtype or meta["in_dtype"] != self.in_dtype:
                 raise ValueError("readout part dtypes do not match this plan")
-        workers = workers or min(16, os.cpu_count() or 1)
-        with ThreadPoolExecutor(max(1, workers)) as pool:
-            blobs = list(pool.map(lambda part: rtc_compile(part[0]), parts))
+        blobs = rtc_compile_many([part[0] for part in parts], workers)
         n = len(parts)
         self._readout_part_code = [ctypes.create_string_buffer(b, len(b)) for b in blobs]
         codes = (_vp * n)(*[ctypes.cast(c, _vp) for c in self._readout_part_code])
