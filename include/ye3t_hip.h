@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define YE3T_HIP_ABI_VERSION 61 /* reference native ABI floor is 42 (execution_plan.py:35) */
+#define YE3T_HIP_ABI_VERSION 62 /* reference native ABI floor is 42 (execution_plan.py:35) */
 
 typedef struct ihipStream_t* ye3t_stream_t; /* == hipStream_t */
 
@@ -188,6 +188,11 @@ int ye3t_hip_ace_density_forward(const ye3t_density_args* args, void* A, ye3t_st
 /* Name of the kernel the last ye3t_hip_ace_density_forward call on this thread
  * launched ("" if none), for profiling.  No reference counterpart. */
 const char* ye3t_hip_last_density_kernel(void);
+
+/* Name of the library's own kernel that a call on this thread launched last (""
+ * if none; generated kernels are not counted), for tests of a dispatch and for
+ * profiling.  No reference counterpart. */
+const char* ye3t_hip_last_kernel(void);
 
 /* Edge-vector gradient of the fused stage 1 (forces): edge_gradient[e, :] =
  * d <density_adjoint, A> / d edge_vectors[e, :] for density_adjoint shaped like

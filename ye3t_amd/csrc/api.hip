@@ -11,9 +11,11 @@ namespace ye3t {
 namespace {
 thread_local std::string g_last_error;
 thread_local const char* g_last_density_kernel = "";
+thread_local const char* g_last_kernel = "";
 }
 
 void set_density_kernel(const char* name) { g_last_density_kernel = name; }
+void set_last_kernel(const char* name) { g_last_kernel = name; }
 
 int set_error(int code, const char* fmt, ...) {
   char buf[1024];
@@ -714,6 +716,8 @@ int ye3t_hip_has_cpu(void) { return 0; }
 const char* ye3t_hip_last_error(void) { return g_last_error.c_str(); }
 
 const char* ye3t_hip_last_density_kernel(void) { return g_last_density_kernel; }
+
+const char* ye3t_hip_last_kernel(void) { return g_last_kernel; }
 
 int ye3t_hip_device_caps(int device, ye3t_hip_caps* out) {
   YE3T_REQUIRE(out != nullptr, "caps output is NULL");

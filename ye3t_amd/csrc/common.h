@@ -16,6 +16,8 @@ int set_error(int code, const char* fmt, ...);
 void clear_error();
 // records the kernel an ace_density_forward call launched (static string)
 void set_density_kernel(const char* name);
+// records the kernel that was launched last on this thread (static string)
+void set_last_kernel(const char* name);
 
 #define YE3T_CHECK_HIP(expr)                                                              \
   do {                                                                                    \
@@ -33,6 +35,7 @@ void set_density_kernel(const char* name);
 inline int check_launch(const char* what) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(YE3T_ELAUNCH, "%s launch failed: %s", what, hipGetErrorString(e));
+  set_last_kernel(what);
   return YE3T_OK;
 }
 

@@ -990,7 +990,7 @@ int fa_launch(const ye3t_hip_factorized_angular_plan* p, int op, const void* pac
                          static_cast<const T*>(packed), static_cast<const T*>(gout), static_cast<const T*>(weight),
                          batch, units, static_cast<T*>(out));
     }
-    return check_launch("factorized_angular");
+    return check_launch(op == 0 ? "fa_sorted_forward_kernel" : "fa_sorted_adjoint_kernel");
   }
   const int spw = fa_samples_per_wave(p, copies);
   if (spw == 0)
@@ -1018,7 +1018,7 @@ int fa_launch(const ye3t_hip_factorized_angular_plan* p, int op, const void* pac
                        static_cast<const T*>(packed), static_cast<const T*>(gout), static_cast<const T*>(weight),
                        batch, spw, static_cast<T*>(out));
   }
-  return check_launch("factorized_angular");
+  return check_launch(op == 0 ? "fa_forward_kernel" : op == 2 ? "fa_linear_kernel" : "fa_adjoint_kernel");
 }
 
 int fa_dispatch(const ye3t_hip_factorized_angular_plan* p, int op, const void* packed, const void* gout,

@@ -12,7 +12,7 @@ import numpy as np
 
 _PKG = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.path.join(_PKG, "libye3t_hip.so")
-ABI_VERSION = 61
+ABI_VERSION = 62
 _LIB = None
 
 F32, F64 = 0, 1
@@ -105,6 +105,7 @@ def lib():
     L.ye3t_hip_has_cpu.restype = ctypes.c_int
     L.ye3t_hip_last_error.restype = ctypes.c_char_p
     L.ye3t_hip_last_density_kernel.restype = ctypes.c_char_p
+    L.ye3t_hip_last_kernel.restype = ctypes.c_char_p
     L.ye3t_hip_device_caps.argtypes = [ctypes.c_int, ctypes.POINTER(Caps)]
     L.ye3t_hip_radial_table.argtypes = [ctypes.c_int, _vp, _vp, _vp, _i64, _i64, _vp, _vp, _vp]
     L.ye3t_hip_real_sph_table.argtypes = [ctypes.c_int, _vp, _i64, _i64, ctypes.c_double, _vp, _vp, _vp]
@@ -233,7 +234,7 @@ EXPORTED_SYMBOLS = (
     "ye3t_hip_symmetric_power_shared_sparse_monomial_adjoint",
     "ye3t_hip_symmetric_power_shared_sparse_monomial_double_backward", "ye3t_hip_code_object_kernel_info",
     "ye3t_hip_part_private_limit", "ye3t_hip_check_indices",
-    "ye3t_hip_csr_offsets", "ye3t_hip_position_bounds",
+    "ye3t_hip_csr_offsets", "ye3t_hip_position_bounds", "ye3t_hip_last_kernel",
 )
 
 
@@ -566,6 +567,11 @@ def ace_density_edge_gradient(density_adjoint, edge_vectors, row_offsets, neighb
 def last_density_kernel():
     """Kernel launched by the last ``ace_density_forward`` call on this thread."""
     return lib().ye3t_hip_last_density_kernel().decode()
+
+
+def last_kernel():
+    """The library's own kernel launched last on this thread (generated kernels are not counted)."""
+    return lib().ye3t_hip_last_kernel().decode()
 
 
 def _host_i64(a):
