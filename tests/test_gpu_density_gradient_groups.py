@@ -97,7 +97,7 @@ def test_uneven_structures(gpu, mode, channels, degrees):
     d, kw = _device(inp, "f64", gpu)
     got = native.ace_density_edge_gradient(torch.as_tensor(gA, device=gpu), d["edge_vectors"], d["row_offsets"],
                                            d["neighbors"], **kw)
-    assert E * 16 * 49 >= 7.5e7 and E // 4 >= len(counts) * channels
+    assert native.last_kernel() == "density_edge_gradient_mfma_kernel"
     err = column_rel_error(got.cpu().numpy(), oracle.ace_density_edge_gradient(inp, gA))
     flush(f"  {err:.2e}")
     assert err < TOL["f64"]
@@ -114,12 +114,44 @@ def test_radial_rows(gpu, n_max, channels, dtypes):
 
     inp = _workload("species" if channels > 1 else "single", 4500 if channels == 1 else 1500, 100, 97, n_max, 6, channels)
     shape = (inp["atom_count"], channels, n_max + 1, 49)
-    assert inp["edge_count"] * (n_max + 1) * 49 >= (7.5e7 if channels == 1 else 2.5e7)
     d, kw = _device(inp, dtypes[0], gpu)
     gd = torch.as_tensor(np.random.default_rng(98).normal(size=shape), device=gpu)
     gd = gd.to(torch.float64 if dtypes[1] == "f64" else torch.float32)
     got = native.ace_density_edge_gradient(gd, d["edge_vectors"], d["row_offsets"], d["neighbors"], **kw).cpu().numpy()
+    assert native.last_kernel() == "density_edge_gradient_mfma_kernel"
     ref = oracle.ace_density_edge_gradient(rounded_inputs(inp, dtypes[0]), gd.double().cpu().numpy())
     err = _error(got, ref)
     flush(f"  {err:.2e}")
     assert err < TOL[dtypes[0]]
+
+
+@pytest.mark.parametrize("channels,atoms,degree,n_max,l_max,grouped", [
+    (2, 3000, 60, 6, 6, True), (2, 3000, 60, 5, 6, False),       # seven radial rows, six
+    (4, 4500, 36, 12, 4, True), (5, 4500, 36, 12, 4, False),     # four edges a group and above, below
+    (2, 2200, 60, 15, 4, True), (2, 2150, 60, 15, 4, False),     # 65 536 edges, fewer
+    (1, 2200, 150, 9, 6, True), (1, 2200, 150, 8, 6, False),     # one channel: 7.5e7 values to gather, fewer
+    (2, 2300, 60, 14, 4, True), (2, 2300, 60, 13, 4, False),     # 2.5e7 of them, fewer
+    (2, 3500, 60, 15, 3, False), (2, 2300, 60, 15, 7, False),    # l_max
+])
+def test_both_sides_of_the_rule(gpu, channels, atoms, degree, n_max, l_max, grouped):
+    """The kernel that a call goes to at each line of the rule, and its values there."""
+    flush(f"edge gradient rule: {channels} channels, {atoms} x {degree}, n_max {n_max}, l_max {l_max}")
+    import torch
+
+    from ye3t_amd.runtime import native
+
+    inp = _workload("species" if channels > 1 else "single", atoms, 0, 99, n_max, l_max, channels)
+    rng = np.random.default_rng(100)
+    E = atoms * degree // 2
+    vec = rng.normal(size=(E, 3))
+    counts = np.full(atoms, degree // 2)
+    inp.update(edge_count=E, centers=np.repeat(np.arange(atoms), counts),
+               row_offsets=np.concatenate([[0], np.cumsum(counts)]).astype(np.int64),
+               neighbors=rng.integers(0, atoms, E),
+               edge_vectors=vec / np.linalg.norm(vec, axis=1, keepdims=True) * rng.uniform(0.5, 5.3, (E, 1)))
+    gA = rng.normal(size=(atoms, channels, n_max + 1, (l_max + 1) ** 2))
+    d, kw = _device(inp, "f64", gpu)
+    got = native.ace_density_edge_gradient(torch.as_tensor(gA, device=gpu), d["edge_vectors"], d["row_offsets"],
+                                           d["neighbors"], **kw)
+    assert native.last_kernel() == ("density_edge_gradient_mfma_kernel" if grouped else "density_edge_gradient_kernel")
+    assert column_rel_error(got.cpu().numpy(), oracle.ace_density_edge_gradient(inp, gA)) < TOL["f64"]

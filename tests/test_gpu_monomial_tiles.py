@@ -92,3 +92,33 @@ def test_grouped_values_scale_their_monomials(gpu, dtype, big):
     want = [12 * big ** 2, -4 * big ** 2 - 12 * big]
     assert torch.allclose(gx.double(), torch.tensor([want] * 3, device=gpu, dtype=torch.float64),
                           rtol=1e-14 if dtype == "f64" else 1e-6, atol=0)
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("exponents", [(15, 15), (16, 1), (17, 31), (0, 300)])
+def test_exponents_beyond_four_bits(gpu, dtype, exponents):
+    """Tables whose exponents are packed into four bits each, and, one too large, tables that are not."""
+    flush(f"monomial tiles, exponents {exponents}, {dtype}")
+    import torch
+
+    from ye3t_amd import runtime
+
+    rng = np.random.default_rng(sum(exponents))
+    counts = np.array([[exponents[0], 0, 2], [0, exponents[1], 1], [1, 1, 0]])
+    offs, outs, terms, vals = np.array([0, 2, 4]), np.array([0, 0, 1, 1]), np.array([0, 1, 2, 1]), rng.normal(size=4)
+    real = torch.float64 if dtype == "f64" else torch.float32
+    x = torch.as_tensor(rng.uniform(0.95, 1.05, (67, 3)) * rng.choice([-1, 1], (67, 3)), device=gpu).to(real)
+    g = torch.as_tensor(rng.normal(size=(67, 2)), device=gpu).to(real)
+    xr, gr, vr = x.double().cpu().numpy(), g.double().cpu().numpy(), torch.as_tensor(vals).to(real).double().numpy()
+    want = oracle.symmetric_power_shared_monomial(xr, counts, offs, terms, vr)
+    grad = oracle.symmetric_power_shared_monomial_adjoint(gr, xr, counts, offs, terms, vr)
+    for name, table in (("monomial", (counts[terms], offs, outs, vals)), ("shared_monomial", (counts, offs, terms, outs, vals))):
+        xs = x.clone().requires_grad_(True)
+        out = getattr(runtime, f"symmetric_power_{name}_contraction")(xs, *table)
+        (gx,) = torch.autograd.grad(out, xs, g)
+        # a power e by squaring carries up to e roundings (each squaring doubles those before it), the other
+        # factors and the sum less than eight; a column's largest value is at most sqrt(67) its root mean square
+        bound = (max(exponents) + 8) * (2.0 ** -53 if dtype == "f64" else 2.0 ** -24) * 67 ** 0.5
+        errs = column_rel_error(out.detach().cpu().numpy(), want), column_rel_error(gx.cpu().numpy(), grad)
+        flush(f"  {name} {errs[0]:.2e} {errs[1]:.2e} of {bound:.2e}")
+        assert max(errs) < bound
