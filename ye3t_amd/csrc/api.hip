@@ -98,7 +98,7 @@ __device__ inline void copy_rows(const Real* __restrict__ tile, int rows, Real* 
 }
 
 // Radial table: lane = edge, one Chebyshev pass over n.  128 edges a
-// workgroup: 32 KB of tile at 16 fp64 values and derivatives, five workgroups
+// workgroup: 34 KB of tile at 16 fp64 values and derivatives, four workgroups
 // in a compute unit.
 constexpr int kRadialRows = 128;
 

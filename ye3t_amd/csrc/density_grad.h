@@ -1,6 +1,7 @@
 // What the edge-gradient kernels of the stage-1 density share: their
-// parameters, and the harmonics and their contracted gradient with compile-time
-// bounds.
+// parameters and the harmonics with compile-time bounds; and the harmonics'
+// contracted gradient of the lane-per-edge kernel (the grouped one reads its
+// factors from a tile).
 #pragma once
 
 #include "common.h"
@@ -26,9 +27,10 @@ struct GradParams {
 };
 
 // Y_k(u) for k < (LMAX + 1)^2 (the reference's real SH, same recurrence as
-// real_sph_row) with compile-time bounds, so Y stays in registers.
+// real_sph_row) with compile-time bounds, so Y stays in registers, or goes to a
+// row of a tile.
 template <int LMAX>
-__device__ inline void sph_values(double x, double y, double z, const NormTable& nt, double* Y) {
+__device__ inline void sph_values(double x, double y, double z, const NormTable& nt, double* __restrict__ Y) {
   const double sqrt2 = 1.4142135623730950488016887242096981;
   double cr = 1.0, ci = 0.0, qmm = 1.0;
 #pragma unroll

@@ -206,46 +206,6 @@ __device__ inline GmEdge<In> gm_edge(const GradParams<In, G>& p, const GmChunk& 
 }
 
 
-// Y_k(u) into a row of the tile.
-template <int LMAX>
-__device__ inline void gm_values(double x, double y, double z, const NormTable& nt, double* __restrict__ row) {
-  const double sqrt2 = 1.4142135623730950488016887242096981;
-  double cr = 1.0, ci = 0.0, qmm = 1.0;
-#pragma unroll
-  for (int m = 0; m <= LMAX; ++m) {
-    if (m > 0) {
-      qmm *= double(2 * m - 1);
-      const double nr = cr * x - ci * y;
-      const double ni = cr * y + ci * x;
-      cr = nr;
-      ci = ni;
-    }
-    double q2 = 0.0, q1 = 0.0;
-#pragma unroll
-    for (int l = m; l <= LMAX; ++l) {
-      double q;
-      if (l == m) {
-        q = qmm;
-      } else if (l == m + 1) {
-        q = double(2 * m + 1) * z * qmm;
-      } else {
-        q = (double(2 * l - 1) * z * q1 - double(l + m - 1) * q2) * nt.inv[l - m];
-      }
-      q2 = q1;
-      q1 = q;
-      const double n = nt.v[l * (kMaxL + 1) + m];
-      const int base = l * l + l;
-      if (m == 0) {
-        row[base] = n * q;
-      } else {
-        const double s = sqrt2 * n * q;
-        row[base + m] = s * cr;
-        row[base - m] = -s * ci;
-      }
-    }
-  }
-}
-
 // sum_k t_k grad_u Y_k(u) (sph_gradient_dot's sum, t read from a row of the tile).
 template <int LMAX>
 __device__ inline void gm_gradient(double x, double y, double z, const NormTable& nt, const double* __restrict__ t,
@@ -512,7 +472,7 @@ density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, GmShares
         }
       }
     }
-    if (valid) gm_values<LMAX>(ux, uy, uz, p.nt, Yt[col]);
+    if (valid) sph_values<LMAX>(ux, uy, uz, p.nt, Yt[col]);
     gm_wave_sync();
 
     // ---- products, group by group

@@ -465,8 +465,8 @@ def ace_density_forward(edge_vectors, row_offsets, neighbors, *, atom_count, cha
     ``accumulate_dtype`` (default: ``out_dtype``) is the type of the
     accumulation: float64 with a float32 ``A`` accumulates in fp64 and rounds
     each density value once to fp32.  ``validate`` range-checks the CSR
-    offsets, neighbour and species indices first (one device reduction and a
-    scalar read-back each); a caller that has already validated these inputs
+    offsets, neighbour and species indices first (one kernel and one wait,
+    :func:`check_indices`); a caller that has already validated these inputs
     may skip it.
     """
     import torch
@@ -635,12 +635,6 @@ def check_shared_table(D, monomial_counts, output_offsets, coefficient_terms, co
     if np.any(counts < 0):
         raise ValueError("monomial_counts must be nonnegative")
     return counts, offs, terms, outs
-
-
-def _dev_i64(a, device):
-    import torch
-
-    return torch.as_tensor(a, dtype=torch.int64, device=device).contiguous()
 
 
 def _upload(device, dtype, values, *ints):
