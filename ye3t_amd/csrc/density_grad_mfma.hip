@@ -21,8 +21,8 @@
 //            species and 48 neighbours); t replaces Y in LDS;
 //   chain    lane = edge: the gradient of the harmonics contracted with t.
 // Measured (events): 8 species, n_max 12, l_max 6, 30 000 atoms x 48: 691 us for
-// the lane-per-edge kernel, 470 us here; 4 species, n_max 10, l_max 4,
-// 20 000 x 32: 121 and 100 us.  It is bound by one wave per SIMD
+// the lane-per-edge kernel, 465 us here; 4 species, n_max 10, l_max 4,
+// 20 000 x 32: 121 and 97 us.  It is bound by one wave per SIMD
 // (two at l_max 4) working through dependent fp64 instructions: the tile, 40 KB
 // at l_max 6, limits how many are resident.  Without the block loads it takes
 // 469 us, without the products 161.  Four waves sharing a tile, each with a
@@ -157,16 +157,15 @@ __device__ inline GmChunk gm_take(const GradParams<In, G>& p, int64_t a, int64_t
   GmChunk c;
   c.a = a;
   c.e = e;
-  const int left = e_end - e < 65 ? int(e_end - e) : 65;
-  const int64_t rel = (a + 1 + lane < p.N && window < e_end ? window : e_end) - e;
-  c.end = rel < 0 ? 0 : (rel > 65 ? 65 : int(rel));
-  const uint64_t fits = gm_ballot(a + 1 + lane <= p.N && c.end <= 64);
-  const uint64_t before = gm_ballot(c.end < left);
-  // both are prefixes (the offsets rise); the atom after those that end before the wave does is its last
-  const int nf = ~fits == 0 ? 64 : __builtin_ctzll(~fits);
-  const int nb = ~before == 0 ? 64 : __builtin_ctzll(~before) + 1;
-  c.na = left <= 0 ? 0 : (nf < nb ? nf : nb);
-  c.cnt = c.na > 0 ? __builtin_amdgcn_readlane(c.end, c.na - 1) : (left <= 0 ? 0 : (left < 64 ? left : 64));
+  const int most = e_end - e < 65 ? int(e_end - e) : 65;
+  const int64_t rel = window - e;
+  c.end = rel < 0 ? 0 : (rel > most || a + 1 + lane >= p.N ? most : int(rel));
+  const uint64_t before = gm_ballot(c.end < most);
+  // a prefix (the offsets rise): the atoms that fit a chunk, or, where the wave
+  // ends in this one, those before its last
+  const int n = ~before == 0 ? 64 : __builtin_ctzll(~before);
+  c.na = most == 65 ? n : (most <= 0 ? 0 : (n < 64 ? n + 1 : 64));
+  c.cnt = c.na > 0 ? __builtin_amdgcn_readlane(c.end, c.na - 1) : (most <= 0 ? 0 : 64);
   return c;
 }
 
@@ -346,6 +345,9 @@ density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, GmShares
                             ? p.E
                             : gm_bound(keys[1], shares.per_atom, atoms[1], first_after, last_after, p.E);
   if (e_begin >= e_end) return;
+  // the lane's row in the last step (the steps before it are full, launch_shape).  Rows past the
+  // model's last meet a zero adjoint, but may hold no number themselves (0 / 0 at lambda 0): its last stands in
+  const int last = 4 * (KS - 1) + kq < p.nr ? 4 * (KS - 1) + kq : p.nr - 1;
   const int64_t block = int64_t(p.nr) * LW;
   const unsigned voff = unsigned(kq * LW + cc) * unsigned(sizeof(G));
   auto channel = [&](const GmEdge<In>& edge) {
@@ -407,9 +409,7 @@ density_edge_gradient_mfma_kernel(GradParams<In, G> p, GmRadial radial, GmShares
       for (int ct = 0; ct < CT; ++ct) t[ct] = u[ct] = 0.0;
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        // rows past the model's last meet a zero adjoint, but may hold no number themselves (0 / 0 at
-        // lambda 0, where rows 0 and 1 are well defined): the last row stands in for them
-        const int n = 4 * s + kq < p.nr ? 4 * s + kq : p.nr - 1;
+        const int n = s + 1 < KS ? 4 * s + kq : last;
         const double ar = At[n][ci], ad = At[NRC + n][ci];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
@@ -549,6 +549,7 @@ int gm_waves() {
 
 template <int LMAX, int NRC, typename In, typename G>
 int launch_shape(const GradParams<In, G>& p, hipStream_t s) {
+  if (p.nr > NRC || p.nr <= (NRC - 1) / 4 * 4) return YE3T_EUNSUPPORTED;  // all but the last step full
   static const int per_cu = gm_waves<LMAX, NRC, In, G>();  // the kernel's own, the same on every gfx950
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
