@@ -596,11 +596,12 @@ __global__ __launch_bounds__(256) void csr_offsets_kernel(const int64_t* __restr
 // vectors of the edge rows with every step's read requested before the first
 // write; the output is streamed with non-temporal stores (written once, not
 // re-read here).  Centres are validated by the caller; an index outside [0, N)
-// is clamped so that no access leaves the array.  Several steps where the copies
+// is clamped so that no access leaves the array.  Eight steps where the copies
 // do not fit the caches any more, one where more workgroups count: fp64, 144
-// channels, 240 000 edges (17 million vectors) 60 us by one step, 45 by four, 51
-// by eight; 20 000 edges (1.4 million) 5.5, 6.3 and 7.5; 225 channels (single
-// values), 100 000 edges (23 million) 53, 45 and 40.
+// channels, 240 000 edges (17 million vectors) after the sums of the same call
+// 92 us by one step, 70 by four, 67 by eight; by itself 20 000 edges (1.4
+// million) 5.5 by one and 7.5 by eight, 225 channels (single values) of 100 000
+// edges (23 million) 53 and 40.
 constexpr int64_t kGatherLarge = 5000000;  // vectors
 
 template <int STEPS, typename Index, typename V>
@@ -635,10 +636,9 @@ __global__ __launch_bounds__(256) void density_adjoint_kernel(const V* __restric
 
 template <typename V>
 int launch_gather(const void* adj, const int64_t* centers, int64_t E, int64_t CV, int64_t N, void* out, hipStream_t s) {
-  constexpr int kSteps = sizeof(V) == 16 ? 4 : 8;
   if (E * CV >= kGatherLarge) {
-    hipLaunchKernelGGL((density_adjoint_kernel<kSteps, int64_t, V>), dim3(grid_for(E * CV, 256 * kSteps)), dim3(256), 0,
-                       s, static_cast<const V*>(adj), centers, E, CV, N, static_cast<V*>(out));
+    hipLaunchKernelGGL((density_adjoint_kernel<8, int64_t, V>), dim3(grid_for(E * CV, 256 * 8)), dim3(256), 0, s,
+                       static_cast<const V*>(adj), centers, E, CV, N, static_cast<V*>(out));
   } else {
     hipLaunchKernelGGL((density_adjoint_kernel<1, uint32_t, V>), dim3(grid_for(E * CV, 256)), dim3(256), 0, s,
                        static_cast<const V*>(adj), centers, E, CV, N, static_cast<V*>(out));
