@@ -81,3 +81,23 @@ def test_monomials_of_2_29_rows(room, form):
     (g,) = torch.autograd.grad(call(x, 1), x, torch.ones((B, 1), device=room))
     assert g[_ends(B)].flatten().tolist() == [6.0, 6.0, 6.0, 6.0, 10.0]
     assert int(g.sum(dtype=torch.float64)) == 6 * (B - 1) + 10
+
+
+def test_channels_of_a_schedule_of_140_million(room):
+    """More parts of a tile than the second grid axis has."""
+    flush("scheduled channels, one edge, 1.4e8 channels")
+    import torch
+
+    from ye3t_amd.runtime import native
+
+    K = 140_000_003
+    one = lambda *s: torch.full(s, 2.0, device=room, dtype=torch.float32)  # noqa: E731
+    zeros = torch.zeros(K, dtype=torch.int64, device=room)
+    scales = torch.full((K,), 3.0, device=room)
+    scales[K - 1] = 5.0
+    values, derivs = native.scheduled_radial_angular_channels(
+        one(1, 1), one(1, 1), one(1, 1), one(1, 1, 3), one(1, 3), torch.zeros(1, dtype=torch.int64, device=room),
+        zeros, zeros, zeros - 1, scales)
+    assert values[0, _ends(K)].tolist() == [12.0, 12.0, 12.0, 12.0, 20.0]
+    assert int(values.sum(dtype=torch.float64)) == 12 * (K - 1) + 20
+    assert int(derivs.sum(dtype=torch.float64)) == 108 * (K - 1) + 180  # 3 scales of (2 2 2 + 2 2)

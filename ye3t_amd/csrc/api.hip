@@ -291,6 +291,7 @@ int launch_channels(const Real* rv, const Real* rd, const Real* av, const Real* 
   part = part < kChannelThreads ? kChannelThreads : (part > 4096 ? 4096 : part);
   int64_t tile = part / K;
   tile = tile < 2 ? 2 : tile / 2 * 2;
+  while (tile * K > part * 65535) part *= 2;  // the second grid axis' limit
   const int64_t parts = tile * K <= part + part / 2 ? 1 : (tile * K + part - 1) / part;
   if (parts == 1) part = tile * K;
   // held: whole edges, and rows of which the channels read most
@@ -303,7 +304,6 @@ int launch_channels(const Real* rv, const Real* rd, const Real* av, const Real* 
   }
   const int64_t groups = (E + tile - 1) / tile;
   YE3T_REQUIRE(fits_grid(groups, kChannelThreads), "too many edges for one launch");  // from 500 GB of rows on
-  YE3T_REQUIRE(parts <= 65535, "too many channels for one launch");
   const dim3 grid{unsigned(groups), unsigned(parts)};
   if (held) {
     hipLaunchKernelGGL((scheduled_channels_kernel<true, Real>), grid, dim3(kChannelThreads),
