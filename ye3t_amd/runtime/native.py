@@ -1052,7 +1052,9 @@ def rtc_compile_many(sources, workers=None):
             except OSError:
                 pass  # no process to be had
 
-        with ThreadPoolExecutor(max(1, min(workers or 12, os.cpu_count() or 1, len(missing)))) as pool:
+        # ranks of one node compile side by side
+        cpus = (os.cpu_count() or 1) // max(1, int(os.environ.get("LOCAL_WORLD_SIZE") or 1))
+        with ThreadPoolExecutor(max(1, min(workers or 12, cpus, len(missing)))) as pool:
             list(pool.map(child, missing))
     return [rtc_compile(src) for src in sources]
 
